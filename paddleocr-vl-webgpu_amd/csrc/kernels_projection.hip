@@ -16,15 +16,13 @@
 // and the hi/lo planes written in the GEMM's tile order (per 128-row tile and
 // 32-wide k step one 16 KiB block [plane][k-chunk (4)][row (128)][8]), so a
 // GEMM stage of the activations is one contiguous 16 KiB run.
-// Kernel 2 (GEMM): 128 x 128 output tiles, K in steps of 32, 4 waves of
-// 64 x 64 (4 x 4 MFMA tiles of v_mfma_f32_16x16x32_f16 each, hi and lo);
-// operand tiles move by direct global-to-LDS loads through a three-stage
-// ring with one barrier per step.  Every load instruction reads long runs:
-// 1 KiB of the activation block, or 16 weight rows x 64 bytes.  Projections
-// with at least 512 tiles of 128 x 256 (gate|up at N=4096) run the wide
-// variant instead (kernel 2b below): 128 x 256 or 128 x 192 tiles, 4 waves,
-// and the tiles of each XCD in one block of the output, so both operands are
-// reused from the XCD's L2.
+// Kernel 2 (GEMM): one template from 128 x 192 down to 16 x 16 output tiles;
+// the host picks the tile by a cost that counts, per compute unit, the matrix
+// time and the bytes through its load path (choose_tile below).  The waves of
+// a workgroup own rows of the tile (activation fragments straight from the
+// planes into registers, no byte read twice) and share its weight columns,
+// which move by direct global-to-LDS loads in whole 128-byte lines; small
+// tiles split the depth over groups of waves.
 
 #include <hip/hip_runtime.h>
 
@@ -39,15 +37,15 @@ namespace {
 
 constexpr int kSplitThreads = 256;
 constexpr int kSplitRows = 8;  // rows per split workgroup: 8 x 16 bytes = one 128-byte line per chunk
-constexpr int kTileM = kProjectionTileRows, kTileN = 128, kTileK = kProjectionStepK;
-constexpr int kGemmThreads = 256;
+constexpr int kTileM = kProjectionTileRows, kTileK = kProjectionStepK;
 constexpr uint32_t kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 constexpr int kTileElems = kTileM * kTileK;  // fp16 elements of one 128 x 32 operand tile
 constexpr int kBlockElems = 2 * kTileElems;  // one activation block: hi and lo planes
-// s_waitcnt immediates (gfx9 encoding: vmcnt bits 3:0, expcnt 6:4, lgkmcnt
-// 11:8, the last two left at their maximum) -- as builtins, so the compiler's
-// own wait insertion knows which loads they retire.
-constexpr int kWaitVm4 = 0x0F74, kWaitVm0 = 0x0F70;  // vmcnt(4) / vmcnt(0)
+// s_waitcnt immediate (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4,
+// lgkmcnt 11:8) -- as builtins, so the compiler's own wait insertion knows
+// which loads they retire.
+constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }  // vmcnt(n), lgkmcnt left at its maximum
+constexpr int kLgkm0 = ~0x0F00;                                                 // mask: lgkmcnt(0) as well
 
 // Exponent e of a row whose largest magnitude is m: m * 2^-e in [2^13, 2^14)
 // (0 for an all-zero row).
@@ -139,28 +137,6 @@ __global__ __launch_bounds__(kSplitThreads) void projection_split_kernel(const f
     }
 }
 
-// LDS layouts.  Activations: the block as stored, [plane][k-chunk (4)][row
-// (128)][8], so the fragment a 16-lane group reads (16 rows, one chunk) is one
-// 256-byte run.  Weights: [row (128)][slot (4)][8] with k-chunk c of row r in
-// slot c ^ ((r / 2) % 4): the 4 slots of a row are one 64-byte run of the
-// weight row (one load of 4 lanes), and the fragment reads (16 rows, one chunk
-// each) have no bank conflicts (measured: SQ_LDS_BANK_CONFLICT 0, against a
-// quarter of the LDS cycles with the swizzle c ^ ((r / 4) % 4)).
-__device__ inline int a_offset(int kchunk, int row) { return (kchunk * kTileM + row) * 8; }
-__device__ inline int w_offset(int kchunk, int row) { return (row * 4 + (kchunk ^ ((row >> 1) & 3))) * 8; }
-
-// Ring stage u of the narrow GEMM: distinct LDS arrays per stage (one
-// function-scope array per instantiation), so the compiler sees that loads
-// into one stage and fragment reads of another do not alias and adds no wait
-// of its own before the reads.
-template <int U> __device__ __forceinline__ uint16_t *ring_a() {
-    __shared__ __align__(16) uint16_t buf[kBlockElems];
-    return buf;
-}
-template <int U, int NT> __device__ __forceinline__ uint16_t *ring_w() {
-    __shared__ __align__(16) uint16_t buf[NT * kTileK];
-    return buf;
-}
 // Calls f(integral_constant<U>) for U = B .. E-1 (compile-time ring indices).
 template <int B, int E> struct StageUnroll {
     template <class F> __device__ __forceinline__ static void run(F &&f) {
@@ -172,235 +148,27 @@ template <int E> struct StageUnroll<E, E> {
     template <class F> __device__ __forceinline__ static void run(F &&) {}
 };
 
-// 128 x NT output tiles (NT = 128 or 160 columns), 4 waves of 64 x NT/2.
-// STAGES-deep ring of (activation block 16 KiB, weight tile NT x 32) stages:
-// step s computes stage s while the loads of stages s+1 .. s+STAGES-1 are in
-// flight.  Three stages (72 or 78 KiB) leave room for two workgroups per
-// compute unit; six (144 KiB, NT = 128) are for launches of at most one
-// workgroup per compute unit, where nothing else on the unit covers the load
-// latency.  NT = 160 serves widths that are multiples of 160 with as many
-// tiles as two workgroups per compute unit hold (q|k|v at N=4096: 512 tiles in
-// one round, against 640 tiles of 128 that leave a second round a quarter
-// full).
-template <int STAGES, int MIN_WGS, int NT>
-__global__ __launch_bounds__(kGemmThreads, MIN_WGS) void projection_gemm_kernel(
-    const uint16_t *__restrict__ tiles, const int32_t *__restrict__ exponents, const uint16_t *__restrict__ weight,
-    const float *__restrict__ bias, float *__restrict__ out, uint32_t rows, uint32_t k_width, uint32_t n_width) {
-    static_assert(NT == 128 || NT == 160, "column tile of 128 or 160");
-    constexpr int CB = NT / 32;                 // 16-column MFMA tiles per wave
-    constexpr int kWLoads = NT == 128 ? 2 : 3;  // weight loads per thread and stage
-    constexpr int kLoads = 4 + kWLoads;         // loads per thread and stage
-    static_assert(STAGES >= 3 && kLoads * (STAGES - 1) <= 63, "vmcnt holds at most 63 outstanding loads");
-    constexpr int kWaitRing = 0x0F70 | (kLoads * (STAGES - 2) & 15) | ((kLoads * (STAGES - 2) >> 4) << 14);
-    constexpr int kWaitRingPrologue = 0x0F70 | (kLoads * (STAGES - 1) & 15) | ((kLoads * (STAGES - 1) >> 4) << 14);
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int row16 = lane & 15, kg = lane >> 4;
-    // XCD-aware tile order: workgroups are dispatched round-robin over the 8
-    // XCDs, so workgroup b runs on XCD b % 8; the permutation below gives XCD
-    // x a contiguous range of tiles in row-major order (whole bands of output
-    // rows), and the L2 of that XCD serves every column tile of its rows.
-    const uint32_t n_tiles = n_width / NT + (n_width % NT != 0);
-    const uint32_t total = gridDim.x, xcd = blockIdx.x % kXcds, idx = blockIdx.x / kXcds;
-    const uint32_t q = total / kXcds, r = total % kXcds;
-    const uint32_t tile = xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
-    const uint32_t mt = tile / n_tiles, m0 = mt * kTileM, n0 = (tile % n_tiles) * NT;
-    const int wm = wave >> 1, wn = wave & 1;  // the wave's 64 x NT/2 part
-    const uint32_t steps = k_width / kTileK;
-    typedef __attribute__((address_space(3))) void *lds_ptr;
-
-    // Direct global-to-LDS loads, 64 lanes x 16 bytes per instruction, lane l
-    // landing at 16 l of the instruction's 1 KiB.  Activations: the 16 KiB
-    // block (tile mt, step s) as 16 instructions of 1 KiB, 4 per wave.
-    // Weights: NT / 16 instructions of 16 rows each; lane l of instruction j
-    // fills LDS slot p = 64 j + l, i.e. row p / 4, slot p % 4.  Wave w issues
-    // instructions 2w and 2w+1 and, for NT = 160, instruction 8 + (w & 1) (so
-    // waves 2 and 3 repeat waves 0 and 1's: the same bytes into the same
-    // place, and every wave counts the same loads).  Weight rows past the end
-    // re-read the last row (never stored).
-    const uint16_t *a_tiles = tiles + static_cast<size_t>(mt) * steps * kBlockElems + (wave * 4) * 512 + lane * 8;
-    const uint32_t last_col = n_width - 1;
-    // (Fixed-size arrays: hipcc's host pass drops the kernel's launch stub,
-    // without a diagnostic, when a lambda called from the generic step lambda
-    // captures a local array whose size depends on the template arguments.)
-    int w_inst[3];
-    size_t w_row_off[3];
-#pragma unroll
-    for (int rw = 0; rw < kWLoads; ++rw) {
-        w_inst[rw] = rw < 2 ? wave * 2 + rw : 8 + (wave & 1);
-        const int p = 64 * w_inst[rw] + lane, wrow = p >> 2;
-        const int kc = (p & 3) ^ ((wrow >> 1) & 3);
-        w_row_off[rw] = static_cast<size_t>(min(n0 + wrow, last_col)) * k_width + kc * 8;
-    }
-    auto stage = [&](uint32_t s, uint16_t *da, uint16_t *dw) {
-        const uint16_t *a = a_tiles + static_cast<size_t>(s) * kBlockElems;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            __builtin_amdgcn_global_load_lds(a + j * 512, (lds_ptr)(da + (wave * 4 + j) * 512), 16, 0, 0);
-#pragma unroll
-        for (int rw = 0; rw < kWLoads; ++rw)
-            __builtin_amdgcn_global_load_lds(weight + w_row_off[rw] + s * kTileK,
-                                             (lds_ptr)(dw + w_inst[rw] * 512), 16, 0, 0);
-    };
-
-    float4_t acc[4][CB];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < CB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-    // 16 x 16 x 32 tiles: A = activations (lane row = l % 16, k = (l / 16) * 8 ..),
-    // B = W^T (lane column = l % 16, same k), C: column l % 16, rows (l / 16) * 4 + i.
-    // A step's 8 + CB fragments (CB weight, 4 hi, 4 lo) are read from LDS
-    // during the previous step's MFMAs (two register sets).
-    struct Frags {
-        half8_t b[CB], h[4], l[4];
-    };
-    auto read_frags = [&](Frags &f, const uint16_t *sa, const uint16_t *sw) {
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-            f.b[cb] = *reinterpret_cast<const half8_t *>(sw + w_offset(kg, wn * (NT / 2) + cb * 16 + row16));
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            const int trow = wm * 64 + rb * 16 + row16;
-            f.h[rb] = *reinterpret_cast<const half8_t *>(sa + a_offset(kg, trow));
-            f.l[rb] = *reinterpret_cast<const half8_t *>(sa + kTileElems + a_offset(kg, trow));
-        }
-    };
-    auto mfmas = [&](const Frags &f) {
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-                acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.h[rb], f.b[cb], acc[rb][cb], 0, 0, 0);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-                acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.l[rb], f.b[cb], acc[rb][cb], 0, 0, 0);
-        }
-    };
-    // Step s (ring slot U = s % STAGES), entered with stage s's fragments in
-    // registers: wait for this thread's loads of stage s+1, finish its
-    // fragment reads of stage s, barrier (every wave's stage s+1 has landed
-    // and nobody reads slot U any more); load stage s+STAGES into slot U
-    // (past the end: the last stage again, never read); then stage s's 8 CB
-    // MFMAs with stage s+1's 8 + CB fragment reads and the kLoads loads
-    // spread among them (sched_group_barrier masks: 0x008 MFMA, 0x100 LDS
-    // read, 0x020 global load).  Unconditional loads keep the waits exact.
-    Frags fa, fb;
-    uint32_t s = 0;
-    auto step = [&](auto uc, Frags &cur, Frags &nxt) {
-        constexpr int U = decltype(uc)::value, N = (U + 1) % STAGES;
-        __builtin_amdgcn_s_waitcnt(kWaitRing & ~0x0F00);  // ... and lgkmcnt(0)
-        __builtin_amdgcn_s_barrier();
-        stage(min(s + U + STAGES, steps - 1), ring_a<U>(), ring_w<U, NT>());
-        read_frags(nxt, ring_a<N>(), ring_w<N, NT>());
-        mfmas(cur);
-        if constexpr (NT == 128) {
-#pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 7, 0);
-        }
-    };
-    // Prologue: stages 0 .. STAGES-1 into every slot, wait for stage 0 (the
-    // other STAGES-1 stages' loads may be outstanding), read its fragments.
-    StageUnroll<0, STAGES>::run([&](auto uc) {
-        constexpr int U = decltype(uc)::value;
-        stage(min(static_cast<uint32_t>(U), steps - 1), ring_a<U>(), ring_w<U, NT>());
-    });
-    __builtin_amdgcn_s_waitcnt(kWaitRingPrologue);
-    __builtin_amdgcn_s_barrier();
-    read_frags(fa, ring_a<0>(), ring_w<0, NT>());
-    // Unrolled by 2 STAGES: the ring slot and the register set are both
-    // compile-time in every step.
-    for (; s + 2 * STAGES <= steps; s += 2 * STAGES) {
-        StageUnroll<0, STAGES>::run([&](auto uc) {
-            if constexpr (decltype(uc)::value % 2 == 0) step(uc, fa, fb); else step(uc, fb, fa);
-        });
-        s += STAGES;
-        StageUnroll<0, STAGES>::run([&](auto uc) {
-            if constexpr ((decltype(uc)::value + STAGES) % 2 == 0) step(uc, fa, fb); else step(uc, fb, fa);
-        });
-        s -= STAGES;
-    }
-    // The remaining < 2 STAGES steps (the fragments of stage s are in fa).
-    StageUnroll<0, STAGES>::run([&](auto uc) {
-        if (s + decltype(uc)::value < steps) {
-            if constexpr (decltype(uc)::value % 2 == 0) step(uc, fa, fb); else step(uc, fb, fa);
-        }
-    });
-    if (s + STAGES < steps) {
-        s += STAGES;
-        StageUnroll<0, STAGES - 1>::run([&](auto uc) {
-            if (s + decltype(uc)::value < steps) {
-                if constexpr ((decltype(uc)::value + STAGES) % 2 == 0) step(uc, fa, fb); else step(uc, fb, fa);
-            }
-        });
-    }
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);  // no load into LDS outlives the loop
-
-    // Epilogue: x 2^e of the row (exact), + bias, f32 stores.
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t r = m0 + wm * 64 + rb * 16 + kg * 4 + i;
-            if (r >= rows) continue;
-            const int e = exponents[r];
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                const uint32_t n = n0 + wn * (NT / 2) + cb * 16 + row16;
-                if (n < n_width) out[static_cast<size_t>(r) * n_width + n] = __builtin_ldexpf(acc[rb][cb][i], e) + bias[n];
-            }
-        }
-    }
+// Slot U of the weight ring: distinct LDS arrays (one function-scope array
+// per instantiation), so the compiler sees that loads into one slot and
+// fragment reads of another do not alias and adds no wait of its own.
+template <int U, int ELEMS> __device__ __forceinline__ uint16_t *weight_ring() {
+    __shared__ __align__(16) uint16_t buf[ELEMS];
+    return buf;
 }
 
-// Kernel 2b (wide projections: enough 128 x 256 output tiles to give every
-// compute unit two): projection_gemm_wide_kernel<NW>, 128 x NW output tiles
-// (NW = 256, or 192 where 192-column tiles fill their rounds of two
-// workgroups per compute unit with fewer columns: gate|up at N=4096), 4 waves
-// of 64 x NW/2 (4 x NW/32 MFMA tiles, hi and lo), K in steps of 32.  The
-// activation stages (16 KiB) move through a three-stage ring, loaded two
-// steps ahead, the weight stages (NW x 64 bytes) through a two-stage ring,
-// loaded one step ahead: 80 (72) KiB, two workgroups per compute unit.  Per
-// 32-wide k step a wave reads 8 activation and NW/32 weight fragments for
-// NW/2 MFMAs, at NW = 256 two thirds of the 128 x 128 kernel's LDS reads per
-// MFMA (12 for 32), and a workgroup stores 32 KiB into LDS for twice the
-// products of the 24 KiB the narrow kernel stores.
-constexpr uint32_t kWideResident = 64;          // workgroups one XCD runs at once (32 compute units x 2)
-
-// Tile order of the wide GEMM.  Workgroup b runs on XCD b % 8, so XCD x
-// takes the workgroups b = 8 i + x and, with them, one block of the output:
-// the row tiles split into 8 / col_groups bands and the column tiles into
-// col_groups bands, col_groups chosen by the host to minimise the operand
-// bytes one XCD reads (a row tile's activations and a column tile's weights
-// are the same size).  Inside the block, generations of `gen` columns: all
-// row tiles of the block for columns [g gen, g gen + gen), row-major, so the
-// workgroups resident at once share both operands in the XCD's L2.
-struct WideOrder {
+// Tile order.  Workgroup b runs on XCD b % 8, so XCD x takes the workgroups
+// b = 8 i + x and, with them, one block of the output: the row tiles split
+// into 8 / col_groups bands and the column tiles into col_groups bands.
+// Inside the block, generations of `gen` columns: all row tiles of the block
+// for columns [g gen, g gen + gen), row-major, so the workgroups resident at
+// once share both operands in the XCD's L2.
+constexpr uint32_t kXcdUnits = 32;      // compute units of one XCD
+constexpr uint32_t kXcdResident = 64;   // workgroups one XCD runs at once (two per compute unit)
+struct TileOrder {
     uint32_t row_tiles, col_tiles, col_groups, gen;
 };
 
-__device__ inline bool wide_tile(const WideOrder &o, uint32_t b, uint32_t *mt, uint32_t *nt) {
+__device__ inline bool ordered_tile(const TileOrder &o, uint32_t b, uint32_t *mt, uint32_t *nt) {
     const uint32_t x = b % kXcds, idx = b / kXcds;
     const uint32_t row_groups = kXcds / o.col_groups;
     const uint32_t xr = x / o.col_groups, xc = x % o.col_groups;
@@ -425,171 +193,290 @@ __device__ inline bool wide_tile(const WideOrder &o, uint32_t b, uint32_t *mt, u
     return true;
 }
 
-template <int NW>
-__global__ __launch_bounds__(kGemmThreads, 2) void projection_gemm_wide_kernel(
+// (16 RB RW) x (16 CB) output tiles, RW x KG waves.
+//
+// K group g of KG walks its share of the depth in stages of 64; wave rw of
+// the group owns rows rw 16 RB .. of the tile and every column: per 32-deep
+// half stage it multiplies RB (hi, lo) activation fragments with CB weight
+// fragments.  The activation fragments come straight from the planes (16 rows
+// x 8 k are one 256-byte run) into a ring of AD register sets; no other wave
+// reads them.  The weights of a stage (16 CB rows x 128 bytes) are shared by
+// the group's RW waves through a ring of S LDS slots.
+//
+// Why 64-deep weight stages: a weight row is then read in whole 128-byte
+// lines.  With 32-deep stages every load took half a line, and the compute
+// unit's load path moves lines: L2-resident reads of 16 rows x 64 bytes
+// measured 17 TB/s device-wide against 33 for 8 rows x 128 bytes (direct to
+// LDS or to registers alike), which bound the 128 x 256 and 128 x 160 tile
+// kernels this one replaced.  N=4096, split kernel included, before -> now:
+// q|k|v 55.8 -> 48.3 us, o 52.1 -> 44.8, gate|up 118 -> 93 (1.2 PFLOP/s of
+// MFMAs, the rate of a large bf16 library product on this card), down 69.0
+// -> 62.3.
+//
+// Small launches are bound by latency and by idle compute units, so their
+// tiles are small and the depth is split over KG groups, whose sums are added
+// through LDS in a fixed order (the result does not depend on timing).  211
+// rows: q|k|v 25.3 -> 13.2 us, o 35.8 -> 13.1, gate|up 26.0 -> 15.8, down
+// 47.0 -> 16.7; 16 rows: 18.6 -> 7.7, 29.0 -> 9.2, 18.4 -> 8.1, 40.1 -> 11.3.
+//
+// LDS slot layout [row][8 chunks of 8 k], chunk c of row r in place c ^ (r %
+// 8): a load's 8 lanes still read one line, and the 8 rows of a fragment read
+// fall on distinct 16-byte bank groups.  The last column tile is shifted to
+// end at the last column (n_width >= 16 CB; columns of the overlap are
+// computed twice, bit-identically); CB = 1 serves narrower outputs with
+// clamped weight rows.
+template <int RB, int RW, int CB, int KG, int S, int AD, int MIN_WAVES>
+__global__ __launch_bounds__(RW *KG * 64, MIN_WAVES) void projection_gemm_kernel(
     const uint16_t *__restrict__ tiles, const int32_t *__restrict__ exponents, const uint16_t *__restrict__ weight,
     const float *__restrict__ bias, float *__restrict__ out, uint32_t rows, uint32_t k_width, uint32_t n_width,
-    WideOrder order) {
-    static_assert(NW == 256 || NW == 192, "wide column tile of 256 or 192");
-    constexpr int CB = NW / 32;    // 16-column MFMA tiles per wave
-    constexpr int kWL = NW / 64;   // weight loads (16 rows each) per wave and stage
-    constexpr int kWideElems = NW * kTileK;  // one weight stage: NW rows x 32 k
+    TileOrder order) {
+    typedef int int4_t __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) void *lds_ptr;
+    constexpr int kTM = RB * RW * 16, kTN = CB * 16;
+    constexpr int kStageElems = CB * 1024;           // one K group's weight stage: 16 CB rows x 64 k
+    constexpr int kSlotElems = KG * kStageElems;
+    constexpr int kWLoads = 2 * CB / RW;             // weight loads per wave and stage: 8 rows x 128 bytes each
+    constexpr int kW0 = (kWLoads + 1) / 2;           // of them, issued in the stage's first half
+    constexpr int kALoads = 2 * RB;                  // activation loads per half stage
+    static_assert(kTileM % kTM == 0, "a row tile lies in one 128-row block of the planes");
+    static_assert((2 * CB) % RW == 0, "every wave of a K group loads as much of a stage");
+    static_assert(KG == 1 || (KG - 1) * RW <= 2 * KG, "one ring slot holds the partial sums of a reduction phase");
     uint32_t mt, nt;
-    if (!wide_tile(order, blockIdx.x, &mt, &nt)) return;  // uniform: a smaller block of this XCD
+    if (!ordered_tile(order, blockIdx.x, &mt, &nt)) return;  // uniform: a smaller block of this XCD
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int rw = wave % RW, group = wave / RW;
     const int row16 = lane & 15, kg = lane >> 4;
-    const uint32_t m0 = mt * kTileM, n0 = nt * NW;
-    const int wm = wave >> 1, wn = wave & 1;  // the wave's 64 x NW/2 part: rows wm * 64, columns wn * NW/2
-    const uint32_t steps = k_width / kTileK;
+    const uint32_t m0 = mt * kTM + rw * (RB * 16);
+    const uint32_t n0 = CB == 1 ? nt * kTN : min(nt * kTN, n_width - kTN);
+    const uint32_t steps = k_width / kTileK, stages = (steps + 1) / 2;
+    const uint32_t per_group = (stages + KG - 1) / KG, first = group * per_group;
+    const bool odd = (steps & 1) != 0;  // the last stage has one half
 
-    // The stages as distinct arrays, picked at compile time by the loop
-    // unrolled by six (the period of the two rings).
-    __shared__ uint16_t sa0[kBlockElems], sa1[kBlockElems], sa2[kBlockElems];
-    __shared__ uint16_t sw0[kWideElems], sw1[kWideElems];
-    typedef __attribute__((address_space(3))) void *lds_ptr;
-
-    // Direct global-to-LDS loads, 1 KiB per instruction: activations as in
-    // the narrow kernel (4 per wave); weights NW / 16 instructions of 16 rows,
-    // NW / 64 per wave, lane l of instruction j filling LDS slot p = 64 j + l
-    // (row p / 4, slot p % 4, the row's k-chunk slot ^ ((row / 2) % 4)).
-    // Weight rows past the end re-read the last row (never stored).
-    const uint16_t *a_tiles = tiles + static_cast<size_t>(mt) * steps * kBlockElems + (wave * 4) * 512 + lane * 8;
-    const uint32_t last_col = n_width - 1;
-    // (The per-thread arrays here have fixed sizes, the largest width's, and
-    // only their first kWL / CB entries are used: arrays whose size depends on
-    // the template argument make hipcc's host pass drop the launch stub.)
-    size_t w_row_off[4];
+    const uint16_t *a_base = tiles + static_cast<size_t>(m0 / kTileM) * steps * kBlockElems;
+    const uint32_t a_lane = (kg * kTileM + m0 % kTileM + row16) * 8;
+    // Lane l of a weight load fills LDS place l % 8 of row l / 8 (byte
+    // offsets, which choose_tile keeps within 32 bits; 8-element chunks for CB
+    // = 1, within 32 bits at any depth; w_tail for an odd last stage, whose
+    // second half re-reads the first and is not used).
+    const uint32_t chunk = (lane & 7) ^ (lane >> 3), unit = CB == 1 ? 1 : 16;
+    uint32_t w_lane[2], w_tail[2];
 #pragma unroll
-    for (int rw = 0; rw < kWL; ++rw) {
-        const int p = 64 * (wave * kWL + rw) + lane, wrow = p >> 2;
-        const int kc = (p & 3) ^ ((wrow >> 1) & 3);
-        w_row_off[rw] = static_cast<size_t>(min(n0 + wrow, last_col)) * k_width + kc * 8;
+    for (int j = 0; j < 2; ++j) {
+        const uint32_t r = CB == 1 ? min(j * 8 + static_cast<uint32_t>(lane >> 3), n_width - 1 - n0) : lane >> 3;
+        w_lane[j] = (r * (k_width / 8) + chunk) * unit;
+        w_tail[j] = (r * (k_width / 8) + (chunk & 3)) * unit;
     }
-    auto load_a = [&](uint32_t s, uint16_t *da) {
-        const uint16_t *a = a_tiles + static_cast<size_t>(s) * kBlockElems;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            __builtin_amdgcn_global_load_lds(a + j * 512, (lds_ptr)(da + (wave * 4 + j) * 512), 16, 0, 0);
+    const uint16_t *w_base = weight + static_cast<size_t>(n0) * k_width;
+
+    struct Act {
+        half8_t h[RB], l[RB];
     };
-    auto load_w = [&](uint32_t s, uint16_t *dw) {
+    // Loads past the end re-read the last step or stage (never used), so
+    // every wave has the same loads in flight.
+    auto load_a = [&](uint32_t step, Act &f) {
+        const uint16_t *a = a_base + static_cast<size_t>(min(step, steps - 1)) * kBlockElems;
 #pragma unroll
-        for (int rw = 0; rw < kWL; ++rw)
-            __builtin_amdgcn_global_load_lds(weight + w_row_off[rw] + s * kTileK,
-                                             (lds_ptr)(dw + (wave * kWL + rw) * 512), 16, 0, 0);
+        for (int rb = 0; rb < RB; ++rb) {
+            f.h[rb] = *reinterpret_cast<const half8_t *>(a + a_lane + rb * 128);
+            f.l[rb] = *reinterpret_cast<const half8_t *>(a + kTileElems + a_lane + rb * 128);
+        }
+    };
+    auto load_w = [&](uint32_t stage, uint16_t *slot, int begin, int end) {
+        const uint32_t st = min(stage, stages - 1);
+        const bool tail = odd && st == stages - 1;
+        const uint16_t *w = w_base + static_cast<size_t>(st) * 64;
+#pragma unroll
+        for (int i = begin; i < end; ++i) {
+            const int j = rw * kWLoads + i, q = CB == 1 ? i : 0;
+            const uint32_t lo = tail ? w_tail[q] : w_lane[q];
+            const void *src;
+            if constexpr (CB == 1) src = reinterpret_cast<const half8_t *>(w) + lo;
+            else src = reinterpret_cast<const char *>(w + static_cast<size_t>(j) * 8 * k_width) + lo;
+            __builtin_amdgcn_global_load_lds(src, (lds_ptr)(slot + group * kStageElems + j * 512), 16, 0, 0);
+        }
     };
 
-    float4_t acc[4][8];
+    float4_t acc[RB][CB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < RB; ++a)
 #pragma unroll
         for (int b = 0; b < CB; ++b) acc[a][b] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    // The fragment layouts of the narrow kernel: A = activations (lane row
-    // l % 16, k (l / 16) * 8 ..), B = W^T (lane column l % 16, same k).
-    auto compute = [&](const uint16_t *sa, const uint16_t *sw) {
-        half8_t bf[8];
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-            bf[cb] = *reinterpret_cast<const half8_t *>(sw + w_offset(kg, wn * (NW / 2) + cb * 16 + row16));
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            const int trow = wm * 64 + rb * 16 + row16;
-            const half8_t ah = *reinterpret_cast<const half8_t *>(sa + a_offset(kg, trow));
-            const half8_t al = *reinterpret_cast<const half8_t *>(sa + kTileElems + a_offset(kg, trow));
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-                acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bf[cb], acc[rb][cb], 0, 0, 0);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-                acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bf[cb], acc[rb][cb], 0, 0, 0);
+    // Half stage H (compile time, counted from stage `t` of the group): waits
+    // for its operands (the weights of a stage by vmcnt and, with several
+    // waves in the group, the barrier that also frees the slot of the stage
+    // before; the fragments by the compiler's own wait), reads the weight
+    // fragments, issues its half of the weight loads of stage +S-1 and the
+    // activation loads of half stage +AD-1, then its 2 RB CB MFMAs (16 x 16 x
+    // 32: A = activations, lane row l % 16, k (l / 16) * 8 ..; B = W^T, lane
+    // column l % 16, same k).  The scheduling barriers keep the loads ahead of
+    // the MFMAs: left alone the compiler sinks them to the end of the stage,
+    // right before the next wait.
+    // Outstanding loads allowed: at a stage's start everything issued after
+    // its last weight load, 2 S - 4 half stages and one half's activations.
+    constexpr int kHalfLoads = kALoads + kWLoads / 2;  // (at least)
+    constexpr int kWaitWeights = (2 * S - 4) * kHalfLoads + kALoads, kWaitActs = (AD - 2) * kHalfLoads;
+    constexpr int kWaitStage = kWaitActs < kWaitWeights ? kWaitActs : kWaitWeights;
+    static_assert(S >= 2 && AD >= 2 && kWaitActs <= 63, "vmcnt holds at most 63 outstanding loads");
+    Act f[AD];
+    uint32_t t = 0;
+    auto half = [&](auto hc) {
+        constexpr int H = decltype(hc)::value, kSlot = (H / 2) % S, kNext = (H / 2 + S - 1) % S;
+        const uint32_t st = first + t + H / 2;
+        if constexpr (H % 2 == 0) {
+            __builtin_amdgcn_s_waitcnt(wait_vm(kWaitStage) & kLgkm0);
+            if constexpr (RW > 1) __builtin_amdgcn_s_barrier();
+        } else {
+            __builtin_amdgcn_s_waitcnt(wait_vm(kWaitActs));
         }
-        // Schedule: the weight fragments and the first row block's first,
-        // then each row block's 2 CB MFMAs with the next row block's two
-        // fragment reads issued after its first MFMA and the step's 4 + NW / 64
-        // global-to-LDS loads spread among them (masks: 0x100 LDS read,
-        // 0x008 MFMA, 0x020 global load).  Measured against the compiler's own
-        // order (a wait for each row block's reads): gate|up 138 -> 127 us.
-        __builtin_amdgcn_sched_group_barrier(0x100, CB + 2, 0);
+        const uint16_t *sw = weight_ring<kSlot, kSlotElems>() + group * kStageElems;
+        half8_t b[12];  // the first CB (a fixed size: an array whose size depends on the template arguments,
+                        // captured in a generic lambda, makes hipcc's host pass drop the launch stub)
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (rb < 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        for (int cb = 0; cb < CB; ++cb) {
+            const int r = cb * 16 + row16, c = (H % 2) * 4 + kg;
+            b[cb] = *reinterpret_cast<const half8_t *>(sw + (r * 8 + (c ^ (r & 7))) * 8);
+        }
+        load_w(st + S - 1, weight_ring<kNext, kSlotElems>(), H % 2 ? kW0 : 0, H % 2 ? kWLoads : kW0);
+        load_a(2 * st + H % 2 + AD - 1, f[(H + AD - 1) % AD]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (2 * st + H % 2 < steps) {  // uniform
 #pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                __builtin_amdgcn_sched_group_barrier(0x008, (2 * CB - 1) / 3, 0);
-                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+                    acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[H % AD].h[rb], b[cb], acc[rb][cb], 0, 0, 0);
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+                    acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[H % AD].l[rb], b[cb], acc[rb][cb], 0, 0, 0);
             }
-            if constexpr ((2 * CB - 1) % 3 != 0) __builtin_amdgcn_sched_group_barrier(0x008, (2 * CB - 1) % 3, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    // Step s: wait until at most the 4 activation loads of stage s + 1 are
-    // outstanding (this wave's loads of the activations and weights of stage
-    // s have landed), barrier (every wave's have, and every wave has finished
-    // reading the buffers of stage s - 1), load the weights of stage s + 1
-    // and then the activations of stage s + 2 into those buffers (past the
-    // end: the last stage again, never read), compute stage s.  Unconditional
-    // loads keep the waits exact.
-    auto step = [&](uint32_t s, uint16_t *ca, uint16_t *cw, uint16_t *na2, uint16_t *nw1) {
-        __builtin_amdgcn_s_waitcnt(kWaitVm4);
-        __builtin_amdgcn_s_barrier();
-        load_w(min(s + 1, steps - 1), nw1);
-        load_a(min(s + 2, steps - 1), na2);
-        compute(ca, cw);
-    };
-
-    load_a(0, sa0);
-    load_w(0, sw0);
-    load_a(min(1u, steps - 1), sa1);
-    uint32_t s = 0;
-    for (; s + 6 <= steps; s += 6) {
-        step(s, sa0, sw0, sa2, sw1);
-        step(s + 1, sa1, sw1, sa0, sw0);
-        step(s + 2, sa2, sw0, sa1, sw1);
-        step(s + 3, sa0, sw1, sa2, sw0);
-        step(s + 4, sa1, sw0, sa0, sw1);
-        step(s + 5, sa2, sw1, sa1, sw0);
-    }
-    if (s < steps) step(s, sa0, sw0, sa2, sw1);
-    if (s + 1 < steps) step(s + 1, sa1, sw1, sa0, sw0);
-    if (s + 2 < steps) step(s + 2, sa2, sw0, sa1, sw1);
-    if (s + 3 < steps) step(s + 3, sa0, sw1, sa2, sw0);
-    if (s + 4 < steps) step(s + 4, sa1, sw0, sa0, sw1);
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);  // no load into LDS outlives the loop
-
-    // Epilogue: x 2^e of the row (exact), + bias, f32 stores.
+    StageUnroll<0, S - 1>::run([&](auto uc) {
+        constexpr int U = decltype(uc)::value;
+        load_w(first + U, weight_ring<U, kSlotElems>(), 0, kWLoads);
+    });
+    StageUnroll<0, AD - 1>::run([&](auto uc) { load_a(2 * first + decltype(uc)::value, f[decltype(uc)::value]); });
+    __builtin_amdgcn_sched_barrier(0);
+    // The prologue's loads are not in the loop's order: waited for here, so
+    // that the compiler's counts in the loop stay those of the loop.
+    __builtin_amdgcn_s_waitcnt(wait_vm(0));
+    // Unrolled over the period of both rings, so slots and register sets are
+    // compile-time.
+    constexpr int kHalves = 2 * S % AD == 0 ? 2 * S : 2 * S * AD;
+    constexpr uint32_t kPeriod = kHalves / 2;
+    for (; t + kPeriod <= per_group; t += kPeriod) StageUnroll<0, kHalves>::run(half);
+    StageUnroll<0, static_cast<int>(kPeriod) - 1>::run([&](auto uc) {
+        constexpr int U = decltype(uc)::value;
+        if (t + U < per_group) {
+            half(std::integral_constant<int, 2 * U>{});
+            half(std::integral_constant<int, 2 * U + 1>{});
+        }
+    });
+    int4_t ex[RB];
+    float bn[CB];
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
+    for (int rb = 0; rb < RB; ++rb) ex[rb] = *reinterpret_cast<const int4_t *>(exponents + m0 + rb * 16 + kg * 4);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) bn[cb] = bias[min(n0 + cb * 16 + row16, n_width - 1)];
+    __builtin_amdgcn_s_waitcnt(wait_vm(0));  // no load into LDS outlives the loop
+    if constexpr (KG > 1) __syncthreads();   // every wave has read its last stages: the ring is free
+
+    // Row block rb: the groups other than its owner (rb % KG) hand their sums
+    // over through ring slot rb % 2; the owner adds them in the groups' order,
+    // scales by the row's 2^e (exact), adds the bias and stores.  (A slot is
+    // written again two phases later, behind the barrier that its reader
+    // reaches after reading.)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        if constexpr (KG > 1) {
+            const int owner = rb % KG;
+            float4_t *sums = reinterpret_cast<float4_t *>(rb & 1 ? weight_ring<1, kSlotElems>() : weight_ring<0, kSlotElems>());
+            if (group != owner) {
+                float4_t *mine = sums + ((group < owner ? group : group - 1) * RW + rw) * CB * 64 + lane;
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) mine[cb * 64] = acc[rb][cb];
+            }
+            __syncthreads();
+            if (group != owner) continue;  // uniform per wave; every wave reaches every barrier
+#pragma unroll
+            for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) acc[rb][cb] += sums[((g * RW + rw) * CB + cb) * 64 + lane];
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t r = m0 + wm * 64 + rb * 16 + kg * 4 + i;
+            const uint32_t r = m0 + rb * 16 + kg * 4 + i;
             if (r >= rows) continue;
-            const int e = exponents[r];
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb) {
-                const uint32_t n = n0 + wn * (NW / 2) + cb * 16 + row16;
-                if (n < n_width) out[static_cast<size_t>(r) * n_width + n] = __builtin_ldexpf(acc[rb][cb][i], e) + bias[n];
+                const uint32_t n = n0 + cb * 16 + row16;
+                if (n < n_width) out[static_cast<size_t>(r) * n_width + n] = __builtin_ldexpf(acc[rb][cb][i], ex[rb][i]) + bn[cb];
             }
         }
     }
 }
 
-// Order of the wide GEMM's tiles for rows x n_width: the column grouping that
-// minimises the operand bytes of the largest XCD block, and generations of
-// columns sized so that one generation is what an XCD runs at once.
-WideOrder wide_order(uint32_t row_tiles, uint32_t col_tiles) {
-    WideOrder best{row_tiles, col_tiles, 1, 1};
-    uint32_t best_cost = UINT32_MAX;
+// The tiles, largest first.
+struct TileShape {
+    uint32_t rows, cols;
+};
+constexpr TileShape kShapes[] = {{128, 192}, {128, 160}, {128, 128}, {128, 64}, {64, 64}, {32, 64}, {16, 64}, {16, 32}, {16, 16}};
+constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
+
+// Order of the tiles: the column grouping with the smallest largest block
+// (the XCDs finish together), then the fewest operand bytes of that block (a
+// row of activations is twice a row of weights), and generations of columns
+// sized so that one generation is what an XCD runs at once.  *block receives
+// the tiles of the largest block.
+TileOrder tile_order(uint32_t row_tiles, uint32_t col_tiles, const TileShape &t, uint64_t *block) {
+    TileOrder best{row_tiles, col_tiles, 1, 1};
+    uint64_t best_tiles = UINT64_MAX, best_bytes = UINT64_MAX;
     for (uint32_t gc = 1; gc <= kXcds; gc *= 2) {
         const uint32_t gr = kXcds / gc;
-        const uint32_t rb = (row_tiles + gr - 1) / gr, cb = (col_tiles + gc - 1) / gc;
-        if (rb + cb < best_cost) {
-            best_cost = rb + cb;
+        const uint64_t rb = (row_tiles + gr - 1) / gr, cb = (col_tiles + gc - 1) / gc;
+        const uint64_t bytes = rb * t.rows * 2 + cb * t.cols;
+        if (rb * cb < best_tiles || (rb * cb == best_tiles && bytes < best_bytes)) {
+            best_tiles = rb * cb;
+            best_bytes = bytes;
             best.col_groups = gc;
         }
     }
-    const uint32_t rb = (row_tiles + kXcds / best.col_groups - 1) / (kXcds / best.col_groups);
-    best.gen = kWideResident / rb > 0 ? kWideResident / rb : 1;
+    const uint32_t gr = kXcds / best.col_groups, rb = (row_tiles + gr - 1) / gr;
+    best.gen = kXcdResident / rb > 0 ? kXcdResident / rb : 1;
+    *block = best_tiles;
+    return best;
+}
+
+// The tile of a launch: the least clocks of the busiest compute unit per
+// 32-deep step, (tiles it runs) x max(matrix time, load time) with rows cols /
+// 32 clocks of MFMAs (hi and lo, 4096 FLOP per clock) and 2 rows + cols clocks
+// of loads (64 bytes per clock) a tile; the larger tile on ties.  The unit's
+// tiles are those of the largest XCD block over its 32 units.  Against every
+// tile timed at 16 to 4096 rows of the decoder's projections this picks the
+// fastest or one within 3% of it.
+int choose_tile(uint32_t rows, uint32_t k_width, uint32_t n_width, TileOrder *order, uint64_t *block) {
+    int best = kShapeCount - 1;
+    uint64_t best_cost = UINT64_MAX;
+    for (int i = 0; i < kShapeCount; ++i) {
+        const TileShape t = kShapes[i];
+        // The shifted last column tile needs a whole one, and a row of
+        // weights at most 2^29 bytes (32-bit offsets over 8 rows); the 16 x 16
+        // tile takes any.
+        if (i + 1 < kShapeCount && (n_width < t.cols || k_width > 1u << 28)) continue;
+        uint64_t b = 0;
+        const TileOrder o = tile_order((rows + t.rows - 1) / t.rows, n_width / t.cols + (n_width % t.cols != 0), t, &b);
+        const uint64_t mfma = t.rows * t.cols / 32, loads = 2 * t.rows + t.cols;
+        const uint64_t cost = (b + kXcdUnits - 1) / kXcdUnits * (mfma > loads ? mfma : loads);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = i;
+            *order = o;
+            *block = b;
+        }
+    }
     return best;
 }
 
@@ -609,46 +496,27 @@ int launch_linear_projection_f16(const float *input, const uint16_t *weight, con
     default: hipLaunchKernelGGL(projection_split_kernel<0>, split_grid, dim3(kSplitThreads), 0, st, input, rows, k_width, ws.tiles, ws.exponents); break;
     }
     if (hipError_t e = hipGetLastError()) return static_cast<int>(e);
-    const uint32_t cols256 = n_width / 256 + (n_width % 256 != 0), cols192 = n_width / 192 + (n_width % 192 != 0);
-    const uint64_t slots = 2 * kTargetWorkgroups;
-    if (static_cast<uint64_t>(cols256) * m_tiles >= slots) {
-        // Enough wide tiles for two workgroups on every compute unit: the
-        // wide kernel (with fewer, its second slot on most compute units
-        // stays empty, and the narrow kernel's twice as many tiles finish
-        // sooner: q|k|v at N=4096, 320 wide tiles, 80 us against 72).
-        // 192-column tiles where their rounds of two workgroups per compute
-        // unit hold fewer columns than the 256-column tiles' (gate|up at
-        // N=4096: 1024 tiles in two full rounds, against 768 tiles that leave
-        // the second round half empty).
-        const uint64_t rounds256 = (cols256 * m_tiles + slots - 1) / slots, rounds192 = (cols192 * m_tiles + slots - 1) / slots;
-        const bool narrow192 = rounds192 * 192 < rounds256 * 256;
-        const uint32_t wide_cols = narrow192 ? cols192 : cols256;
-        const WideOrder order = wide_order(m_tiles, wide_cols);
-        const uint32_t row_groups = kXcds / order.col_groups;
-        const uint32_t block = ((m_tiles + row_groups - 1) / row_groups) * ((wide_cols + order.col_groups - 1) / order.col_groups);
-        if (narrow192)
-            hipLaunchKernelGGL(projection_gemm_wide_kernel<192>, dim3(kXcds * block), dim3(kGemmThreads), 0, st,
-                               ws.tiles, ws.exponents, weight, bias, out, rows, k_width, n_width, order);
-        else
-            hipLaunchKernelGGL(projection_gemm_wide_kernel<256>, dim3(kXcds * block), dim3(kGemmThreads), 0, st,
-                               ws.tiles, ws.exponents, weight, bias, out, rows, k_width, n_width, order);
-        return static_cast<int>(hipGetLastError());
+    TileOrder order;
+    uint64_t block = 0;
+    const int shape = choose_tile(rows, k_width, n_width, &order, &block);
+    const dim3 grid(static_cast<uint32_t>(kXcds * block));
+#define PVLC_PROJECTION_LAUNCH(RB, RW, CB, KG, S, AD, MW)                                                          \
+    do {                                                                                                           \
+        hipLaunchKernelGGL((projection_gemm_kernel<RB, RW, CB, KG, S, AD, MW>), grid, dim3((RW) * (KG) * 64), 0, st, \
+                           ws.tiles, ws.exponents, weight, bias, out, rows, k_width, n_width, order);              \
+    } while (0)
+    switch (shape) {  // kShapes
+    case 0: PVLC_PROJECTION_LAUNCH(2, 4, 12, 1, 3, 3, 2); break;
+    case 1: PVLC_PROJECTION_LAUNCH(2, 4, 10, 1, 3, 3, 2); break;
+    case 2: PVLC_PROJECTION_LAUNCH(2, 4, 8, 1, 3, 3, 2); break;
+    case 3: PVLC_PROJECTION_LAUNCH(2, 4, 4, 2, 3, 3, 2); break;
+    case 4: PVLC_PROJECTION_LAUNCH(2, 2, 4, 2, 3, 3, 2); break;
+    case 5: PVLC_PROJECTION_LAUNCH(2, 1, 4, 4, 2, 4, 2); break;
+    case 6: PVLC_PROJECTION_LAUNCH(1, 1, 4, 4, 2, 4, 2); break;
+    case 7: PVLC_PROJECTION_LAUNCH(1, 1, 2, 8, 2, 4, 4); break;
+    default: PVLC_PROJECTION_LAUNCH(1, 1, 1, 8, 2, 4, 4); break;
     }
-    const uint32_t tiles = (n_width / kTileN + (n_width % kTileN != 0)) * m_tiles;  // < 2^24 (checked by the caller)
-    const uint32_t tiles160 = (n_width / 160 + (n_width % 160 != 0)) * m_tiles;
-    if (tiles <= kTargetWorkgroups) {
-        // One workgroup per compute unit at most: the six-stage ring.
-        hipLaunchKernelGGL((projection_gemm_kernel<6, 1, 128>), dim3(tiles), dim3(kGemmThreads), 0, st, ws.tiles,
-                           ws.exponents, weight, bias, out, rows, k_width, n_width);
-    } else if (n_width % 160 == 0 && tiles160 <= 2 * kTargetWorkgroups && tiles > 2 * kTargetWorkgroups) {
-        // 160-column tiles fit one round of two workgroups per compute unit
-        // where 128-column tiles need a second.
-        hipLaunchKernelGGL((projection_gemm_kernel<3, 2, 160>), dim3(tiles160), dim3(kGemmThreads), 0, st, ws.tiles,
-                           ws.exponents, weight, bias, out, rows, k_width, n_width);
-    } else {
-        hipLaunchKernelGGL((projection_gemm_kernel<3, 2, 128>), dim3(tiles), dim3(kGemmThreads), 0, st, ws.tiles,
-                           ws.exponents, weight, bias, out, rows, k_width, n_width);
-    }
+#undef PVLC_PROJECTION_LAUNCH
     return static_cast<int>(hipGetLastError());
 }
 
