@@ -271,8 +271,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
     const bool qrope = p.rope_cos != nullptr && qpos >= 0 && static_cast<uint32_t>(qpos) < p.rope_rows;
     float4_t qc[2][2], qs[2][2];  // cos/sin of pairs hk*32 + kg*8 .. +8 (hk = kb & 1)
     {
-        const float *cr = qrope ? p.rope_cos + static_cast<size_t>(qpos) * 64 : reinterpret_cast<const float *>(p.query);
-        const float *sr = qrope ? p.rope_sin + static_cast<size_t>(qpos) * 64 : reinterpret_cast<const float *>(p.query);
+        // Without rotary the loads read the query as a stand-in, in the
+        // operand width that was given (the other pointer is null).
+        const float *stand_in = F32IO ? p.query32 : reinterpret_cast<const float *>(p.query);
+        const float *cr = qrope ? p.rope_cos + static_cast<size_t>(qpos) * 64 : stand_in;
+        const float *sr = qrope ? p.rope_sin + static_cast<size_t>(qpos) * 64 : stand_in;
 #pragma unroll
         for (int hk = 0; hk < 2; ++hk)
 #pragma unroll
