@@ -468,8 +468,9 @@ typedef struct pvlc_hip_paged_prefill_args {
     uint16_t *query_scratch;  /* optional [N][16][128] fp16: receives the rotated query (NULL: not written) */
     uint32_t *error_word;     /* optional: bit 1 = block id out of range (row skipped), bit 2 = position outside the rope table */
     void *workspace;          /* optional, 256-byte aligned, zeroed once (pvlc_hip_workspace_init): split-K schedule
-                                 (long query blocks split over several workgroups and merged); NULL: one workgroup
-                                 per query block.  Launches that share one workspace must be stream-ordered. */
+                                 of long prompts (their long query blocks split over two workgroups and merged);
+                                 NULL, or a shorter prompt: every query block in its own workgroups.  Launches that
+                                 share one workspace must be stream-ordered. */
     uint64_t workspace_bytes; /* at least pvlc_hip_paged_prefill_workspace_bytes(tokens) when workspace is given */
 } pvlc_hip_paged_prefill_args;
 

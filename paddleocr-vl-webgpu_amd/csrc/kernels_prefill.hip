@@ -8,12 +8,21 @@
 // decoder_prefill_mrope_f32 and decoder_kv_append_range_f32
 // (crates/pvlc-wgsl/src/lib.rs:1334-1416).
 //
-// Kernel 2: one workgroup per (16-token query block, kv head) serves the 8
-// query heads of the group; each of its 4 waves owns 2 heads, i.e. two
-// 16-column MFMA tiles of query rows.  Keys and values stream through
-// double-buffered LDS in steps of 64 keys (2 pairs of cache blocks), laid out
-// so every operand read is conflict-free, with the next step loaded into
-// registers while the current one is computed:
+// Kernel 2 (attention) has two forms, chosen in launch_prefill:
+//
+//  * prefill_wave_attention_kernel (prompts up to kPrefillWaveTokens, and any
+//    length without a workspace): one workgroup per (16-token query block, 1
+//    or 2 heads), its waves taking the key steps in turn, each streaming its
+//    keys and values from L2 into registers with no barrier in the loop, and
+//    merging through LDS at the end.  Short prompts have few query blocks, so
+//    the heads and the keys of a block are spread over workgroups and waves.
+//  * prefill_attention_kernel (longer prompts, with a workspace): one
+//    workgroup per (query block or part of one, kv head) serves the 8 query
+//    heads of the group, 2 per wave, over keys and values that stream through
+//    double-buffered LDS in steps of 64 keys, laid out so every operand read
+//    is conflict-free; long blocks split over two workgroups (pair schedule).
+//
+// Both compute
 //   S^T[key][row] = K . Q^T           v_mfma_f32_16x16x32_f16
 //   O[row][dim]  += P[row][key] V      v_mfma_f32_16x16x32_f16
 //   l[row]       += P[row][key] 1      (same MFMA, ones operand)
@@ -21,8 +30,7 @@
 // lane 8 consecutive keys of one tile, which is the P operand of the P.V MFMA.
 // Online softmax in log2 units (scale folded into one FMA per score), the
 // causal mask only on steps that reach the diagonal, and the rescale skipped
-// while the running max is unchanged.  Heavy and light query blocks are
-// paired over the grid for balance.  Replaces
+// while the running max stays near its reference.  Replaces
 // decoder_prefill_gqa_f32 (crates/pvlc-wgsl/src/lib.rs:1262-1332); arithmetic
 // reference causal_gqa_f32 (crates/pvlc-cpu-ref/src/lib.rs:782-853).
 
@@ -43,6 +51,11 @@ constexpr int kKeyStep = 64;     // keys per softmax step (4 cache blocks)
 constexpr int kStepTiles = kKeyStep / 16;
 constexpr int kWaves = 4;        // each wave: 2 of the 8 heads of the group
 constexpr float kLazyRescaleLog2 = 8.0f;  // softmax reference moves only past 2^8
+// Longest prompt of prefill_wave_attention_kernel when the caller gave a
+// workspace for the pair schedule (us, wave / pair: N=3000 f16 63.7 / 66.9,
+// f32 77.6 / 83.0; 3500 80.2 / 75.0, 97.6 / 94.7; 4096 100.5 / 86.0, 124 /
+// 112), and of its one-head form.
+constexpr uint32_t kPrefillWaveTokens = 3072, kPrefillOneHeadTokens = 768;
 
 struct PrefillParams {
     uint32_t tokens;
@@ -61,8 +74,7 @@ struct PrefillParams {
     uint16_t *qrot;
     uint32_t *error_word;
     float scale_log2;
-    // split-K pair schedule (a workspace was given and the blocks are long)
-    bool split;
+    // split-K pair schedule (prefill_attention_kernel)
     uint32_t *counters;  // [pair][kv head]
     float *partials;     // [pair][kv head][2 parts][kPrefillPartialFloats]
     // f32 operands (pvlc_hip_paged_prefill_f32io): query, key, value, output;
@@ -217,33 +229,13 @@ __device__ inline int lds_value_offset(int j, int tile, int half, int dim) {
     return (((j * 2 + tile) * 2 + half) * kHeadDim + dim) * 8;
 }
 
-// Work item b of the grid: query blocks are paired heaviest with lightest,
-// so that the two items a compute unit runs (b and b + qblocks, dispatched
-// in order) sum to about the same number of key steps everywhere.
-__device__ inline void prefill_item(int b, int qblocks, int *qb, uint32_t *g) {
-    if (b < qblocks) {
-        *qb = qblocks - 1 - b;
-        *g = 0;
-    } else {
-        *qb = b - qblocks;
-        *g = 1;
-    }
-}
-
 template <bool F32IO>
 __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(PrefillParams p) {
     const int n = static_cast<int>(p.tokens);
     const int qblocks = (n + kQueryBlock - 1) / kQueryBlock;
     uint32_t g, pair = 0;
     PrefillSegment seg0{}, seg1{};
-    int nseg = 1;
-    if (p.split) {
-        nseg = static_cast<int>(prefill_pair_segments(blockIdx.x, static_cast<uint32_t>(qblocks), &g, &pair, &seg0, &seg1));
-    } else {
-        int qb0;
-        prefill_item(static_cast<int>(blockIdx.x), qblocks, &qb0, &g);
-        seg0 = {static_cast<uint32_t>(qb0), 0u, 1u, 0u, prefill_block_steps(static_cast<uint32_t>(qb0))};
-    }
+    const int nseg = static_cast<int>(prefill_pair_segments(blockIdx.x, static_cast<uint32_t>(qblocks), &g, &pair, &seg0, &seg1));
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int row = lane & 15, kg = lane >> 4;
@@ -767,6 +759,332 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
   if (nseg > 1) run_segment(seg1);
 }
 
+// CT query heads x 16 query tokens per workgroup, KG waves: wave w takes the
+// 32-key steps w, w + KG, .. of the block.  Per step a lane loads its key
+// fragments (2 score MFMAs x 4 dim slices, 16 bytes each, in runs of 128
+// bytes) and value fragments (8 x 16 bytes) of one pair of cache tiles
+// straight into registers, in the operand order of the cache layout; the next
+// step's keys are issued behind this step's score MFMAs and its values behind
+// P.V, so each has most of a step to arrive, and nothing in the loop waits for
+// another wave.  Every wave keeps its own softmax reference; the waves merge
+// in LDS.
+//
+// What bounds it: short prompts by latency (launch, the first loads, the
+// merge; 2 to 4 steps a wave), longer ones by the compute unit's load path:
+// every wave loads all its keys and values, 16 KiB for 34 MFMAs (544 clocks)
+// at 64 bytes per clock.  That is why prompts beyond kPrefillWaveTokens share
+// them through LDS when they have the workspace to split their long blocks.
+// One workgroup per (query block, kv head), as before, kept at most 2 ceil(N /
+// 16) compute units busy, each for the block's whole length: N=211 f16 16.4 ->
+// 9.2 us, 1157 37.5 -> 22.2 (f32 46.8 -> 26.2), 2048 60.2 -> 39.1 (74.7 ->
+// 46.5); without a workspace 4096 109 -> 100 (141 -> 124), 8192 385 -> 347
+// (both kernels' launches included).
+//
+// Workgroup b: kv head b % 2, then the head set, then the query blocks from
+// the last (longest) to the first.  The 16 / CT workgroups of a query block
+// are a multiple of the 8 XCDs, so each XCD reads the keys and values of one
+// kv head only.
+template <bool F32IO, int CT, int KG>
+__global__ __launch_bounds__(KG * 64, 2) void prefill_wave_attention_kernel(PrefillParams p) {
+    constexpr int kHeadSets = kGroup / CT;
+    constexpr int kWaveStep = 32;  // keys per step: one pair of cache tiles
+    const int n = static_cast<int>(p.tokens);
+    const int qblocks = (n + kQueryBlock - 1) / kQueryBlock;
+    const uint32_t g = blockIdx.x & 1u;
+    const int hs = static_cast<int>((blockIdx.x >> 1) % kHeadSets);
+    const int qb = qblocks - 1 - static_cast<int>((blockIdx.x >> 1) / kHeadSets);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int row = lane & 15, kg = lane >> 4;
+    const int t0 = qb * kQueryBlock, my_token = t0 + row;
+    const int nkeys = min(t0 + kQueryBlock, n), last_tile = (nkeys - 1) >> 4;
+    const int steps = (nkeys + kWaveStep - 1) / kWaveStep;
+    const int h0 = static_cast<int>(g) * kGroup + hs * CT;  // first query head
+
+    // Block ids of the wave's tiles, one per lane: lane 2 i + j holds tile j
+    // of the wave's step i0 + i (32 steps a load; a clamped tile past the
+    // end).  Optional arrays are read through the query pointer when they are
+    // not given (at least as long), so no load sits behind a branch.
+    const int32_t *stand_in = F32IO ? reinterpret_cast<const int32_t *>(p.query32) : reinterpret_cast<const int32_t *>(p.query);
+    const int32_t *table = p.block_table ? p.block_table : stand_in;
+    auto tile_of = [&](int i0) { return min(2 * (wave + (i0 + (lane >> 1)) * KG) + (lane & 1), last_tile); };
+    auto tile_id = [&](int t, int32_t b) -> uint32_t {  // an id outside the planes reads block 0
+        if (p.block_table == nullptr) b = t;
+        return b >= 0 && static_cast<uint32_t>(b) < p.num_blocks ? static_cast<uint32_t>(b) : 0u;
+    };
+    const int tq = min(my_token, n - 1);
+    const int32_t id_raw = table[tile_of(0)], pos_raw = (p.positions ? p.positions : stand_in)[tq];
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Raw query: the CT x 2 pairs of 32-dim slices (kb, kb + 2) of a head,
+    // which rotate together, are shared out over the waves.
+    constexpr int kItems = CT * 2, kMine = (kItems + KG - 1) / KG;
+    typedef std::conditional_t<F32IO, float4_t, half8_t> Raw;
+    constexpr int kRawLoads = F32IO ? 2 : 1, kRawElems = F32IO ? 4 : 8;
+    Raw raw[kMine][2][kRawLoads];
+#pragma unroll
+    for (int it = 0; it < kMine; ++it) {
+        const int item = min(wave + it * KG, kItems - 1);
+        const size_t qoff = (static_cast<size_t>(tq) * kQueryHeads + h0 + (item >> 1)) * kHeadDim + (item & 1) * 32 + kg * 8;
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+            for (int f = 0; f < kRawLoads; ++f) {
+                const size_t at = qoff + k2 * 64 + f * kRawElems;
+                if constexpr (F32IO) raw[it][k2][f] = *reinterpret_cast<const Raw *>(p.query32 + at);
+                else raw[it][k2][f] = *reinterpret_cast<const Raw *>(p.query + at);
+            }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t ids = tile_id(tile_of(0), id_raw);
+    const int qpos = p.positions ? pos_raw : tq;
+    const bool qrope = p.rope_cos != nullptr && qpos >= 0 && static_cast<uint32_t>(qpos) < p.rope_rows;
+    float4_t qc[kMine][2], qs[kMine][2];
+    {
+        const float *cr = qrope ? p.rope_cos + static_cast<size_t>(qpos) * 64 : reinterpret_cast<const float *>(stand_in);
+        const float *sr = qrope ? p.rope_sin + static_cast<size_t>(qpos) * 64 : reinterpret_cast<const float *>(stand_in);
+#pragma unroll
+        for (int it = 0; it < kMine; ++it) {
+            const int d0 = (min(wave + it * KG, kItems - 1) & 1) * 32 + kg * 8;
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                qc[it][f] = *reinterpret_cast<const float4_t *>(cr + d0 + f * 4);
+                qs[it][f] = *reinterpret_cast<const float4_t *>(sr + d0 + f * 4);
+            }
+        }
+    }
+    half8_t kf[2][4], vf[8];
+    auto id_of = [&](int i, int j) {
+        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(ids), 2 * (i & 31) + j));
+    };
+    auto load_k = [&](int i) {
+        const uint32_t b0 = id_of(i, 0), b1 = id_of(i, 1);
+        const uint16_t *src = p.key_cache + (static_cast<size_t>(row < 8 ? b0 : b1) * kKvHeads + g) * kBlockHeadElems;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+                kf[h][kb] = *reinterpret_cast<const half8_t *>(src + (kb * 4 + kg) * 128 + (h * 8 + (row & 7)) * 8);
+    };
+    auto load_v = [&](int i) {
+        const uint32_t b0 = id_of(i, 0), b1 = id_of(i, 1);
+        const uint16_t *src = p.value_cache + (static_cast<size_t>(kg < 2 ? b0 : b1) * kKvHeads + g) * kBlockHeadElems;
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            vf[c] = *reinterpret_cast<const half8_t *>(src + (c * 16 + row) * 16 + (kg & 1) * 8);
+    };
+    load_k(0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Rotate (exactly as rotate_chunk does) while the keys and values are in
+    // flight, and share the query fragments (B operand: column = token t0 +
+    // row, dims kb*32 + kg*8 .. +8) through LDS.
+    constexpr int kRow = kHeadDim + 4;  // padded against bank conflicts
+    __shared__ float sm_m[KG][CT * 16], sm_l[KG][CT * 16];
+    __shared__ __align__(16) float sm_o[KG][CT * 16][kRow];
+    half8_t *sm_q = reinterpret_cast<half8_t *>(&sm_o[0][0][0]);  // [head][kb][lane], before the merge
+    static_assert(CT * 4 * 64 * sizeof(half8_t) <= sizeof(sm_o), "the query fragments fit the merge buffer");
+#pragma unroll
+    for (int it = 0; it < kMine; ++it) {
+        const int item = wave + it * KG;
+        if (item < kItems) {
+            half8_t q[2];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float c = qc[it][j >> 2][j & 3], sn = qs[it][j >> 2][j & 3];
+                const float x = static_cast<float>(raw[it][0][j / kRawElems][j % kRawElems]);
+                const float y = static_cast<float>(raw[it][1][j / kRawElems][j % kRawElems]);
+                q[0][j] = to_h(qrope ? x * c + (-y) * sn : x);
+                q[1][j] = to_h(qrope ? y * c + x * sn : y);
+            }
+            sm_q[((item >> 1) * 4 + (item & 1)) * 64 + lane] = q[0];
+            sm_q[((item >> 1) * 4 + (item & 1) + 2) * 64 + lane] = q[1];
+        }
+    }
+    // (fences limited to LDS: the key and value loads stay in flight)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    half8_t qf[CT][4];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) qf[ct][kb] = sm_q[(ct * 4 + kb) * 64 + lane];
+
+    float4_t o[CT][9];  // 8 column tiles of the output, then the row sums
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int c = 0; c < 9; ++c) o[ct][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+    half8_t ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = static_cast<_Float16>(1.0f);
+    const float scale = p.scale_log2;
+    float m_run[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) m_run[ct] = -INFINITY;
+    // Maximum over the 4 lanes of a column (l, l ^ 16, l ^ 32, l ^ 48).
+    auto column_max = [](float c) {
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        u32x2 v = __builtin_amdgcn_permlane16_swap(__float_as_uint(c), __float_as_uint(c), false, false);
+        c = fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+        v = __builtin_amdgcn_permlane32_swap(__float_as_uint(c), __float_as_uint(c), false, false);
+        return fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+    };
+
+    for (int s = wave, i = 0; s < steps; s += KG, ++i) {
+        // The last step of a 32-step block of ids loads the next 32.
+        if (((i + 1) & 31) == 0 && s + KG < steps) ids = tile_id(tile_of(i + 1), table[tile_of(i + 1)]);
+        // Scores: MFMA h leaves lane (column = query token, kg) the keys
+        // (kg & 1)*8 + h*4 + r of the pair's tile kg >> 1.
+        float x[CT][8];
+        {
+            float4_t acc[CT][2];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) acc[ct][h] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        acc[ct][h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[h][kb], qf[ct][kb], acc[ct][h], 0, 0, 0);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[ct][h * 4 + r] = acc[ct][h][r];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(i + 1);  // past the wave's last step: a clamped tile, never used
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + 1 == steps) {  // uniform: the only step that reaches the diagonal or the end of the sequence
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int key = s * kWaveStep + (kg >> 1) * 16 + (kg & 1) * 8 + e;
+                const bool keep = key <= my_token && key < n;
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) x[ct][e] = keep ? x[ct][e] : -INFINITY;
+            }
+        }
+        // Lazy rescale, as in prefill_attention_kernel: the reference moves
+        // when a column's maximum passes it by more than kLazyRescaleLog2
+        // (the first step sets it).
+        bool far = false;
+        float m_new[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            float c = m_run[ct];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c = fmaxf(c, x[ct][e]);
+            m_new[ct] = column_max(c);
+            far |= (m_new[ct] - m_run[ct]) * scale > kLazyRescaleLog2;
+        }
+        if (__any(far)) {  // uniform
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const float alpha = __builtin_amdgcn_exp2f((m_run[ct] - m_new[ct]) * scale);
+                m_run[ct] = m_new[ct];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float a = __shfl(alpha, kg * 4 + r);
+#pragma unroll
+                    for (int c = 0; c < 9; ++c) o[ct][c][r] *= a;
+                }
+            }
+        }
+        // P in fp16; the f32 entry point's weights as the pair hi = fp16(p),
+        // lo = fp16(p - hi) (exact in f32).  A column whose scores are all
+        // -infinity so far has weights 0.
+        half8_t hi[CT], lo[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const float ms = m_run[ct] == -INFINITY ? 0.f : m_run[ct] * scale;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pf = __builtin_amdgcn_exp2f(__builtin_fmaf(x[ct][e], scale, -ms));
+                hi[ct][e] = to_h(pf);
+                if constexpr (F32IO) lo[ct][e] = to_h(pf - static_cast<float>(hi[ct][e]));
+            }
+        }
+#pragma unroll
+        for (int pass = 0; pass < (F32IO ? 2 : 1); ++pass) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    o[ct][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pass ? lo[ct] : hi[ct], vf[c], o[ct][c], 0, 0, 0);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+                o[ct][8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pass ? lo[ct] : hi[ct], ones, o[ct][8], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    // Merge: every wave scales its O and row sums to the common maximum (a
+    // wave without steps holds zeros at -infinity) and stores them; then the
+    // workgroup adds the waves in order, normalises and stores 16-byte chunks.
+    if (kg == 0) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) sm_m[wave][ct * 16 + row] = m_run[ct];
+    }
+    __syncthreads();  // and every wave has read the query fragments
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        float m = sm_m[0][ct * 16 + row];
+#pragma unroll
+        for (int w = 1; w < KG; ++w) m = fmaxf(m, sm_m[w][ct * 16 + row]);
+        const float alpha = __builtin_amdgcn_exp2f((m_run[ct] - m) * scale);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float a = __shfl(alpha, kg * 4 + r);
+            float *dst = sm_o[wave][ct * 16 + kg * 4 + r] + row;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) dst[c * 16] = o[ct][c][r] * a;
+            if (row == 0) sm_l[wave][ct * 16 + kg * 4 + r] = o[ct][8][r] * a;
+        }
+    }
+    __syncthreads();
+    constexpr int kPer = F32IO ? 4 : 8;  // outputs per 16-byte chunk
+    constexpr int kRowChunks = kHeadDim / kPer, kChunks = CT * 16 * kRowChunks;
+    static_assert(kChunks % (KG * 64) == 0, "every thread stores the same number of chunks");
+#pragma unroll
+    for (int j = 0; j < kChunks / (KG * 64); ++j) {
+        const int q = j * (KG * 64) + static_cast<int>(threadIdx.x);  // chunk: [token][head][chunk of the row]
+        const int d0 = q % kRowChunks * kPer, tt = q / kRowChunks / CT, ct = q / kRowChunks % CT;
+        const int r = ct * 16 + tt, t = t0 + tt;
+        float l = 0.f;
+        float4_t v[kPer / 4];
+#pragma unroll
+        for (int e = 0; e < kPer / 4; ++e) v[e] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < KG; ++w) {
+            l += sm_l[w][r];
+#pragma unroll
+            for (int e = 0; e < kPer / 4; ++e) v[e] += *reinterpret_cast<const float4_t *>(&sm_o[w][r][d0 + e * 4]);
+        }
+        const float inv = 1.0f / l;
+        if (t < n) {
+            const size_t off = (static_cast<size_t>(t) * kQueryHeads + h0 + ct) * kHeadDim + d0;
+            if constexpr (F32IO) {
+                *reinterpret_cast<float4_t *>(p.out32 + off) = v[0] * inv;
+            } else {
+                half8_t h;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) h[e] = to_h(v[e >> 2][e & 3] * inv);
+                *reinterpret_cast<half8_t *>(p.out + off) = h;
+            }
+        }
+    }
+}
+
 }  // namespace
 
 int launch_prefill(const pvlc_hip_paged_prefill_args *a, void *stream, const PrefillOperands32 *f32) {
@@ -800,13 +1118,26 @@ int launch_prefill(const pvlc_hip_paged_prefill_args *a, void *stream, const Pre
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return static_cast<int>(e);
     const unsigned qblocks = (a->tokens + kQueryBlock - 1) / kQueryBlock;
-    const PrefillWorkspace ws = prefill_workspace_layout(a->tokens);
-    p.split = a->workspace != nullptr && ws.total > 0;
-    if (p.split) {
-        p.counters = static_cast<uint32_t *>(a->workspace);
-        p.partials = reinterpret_cast<float *>(static_cast<unsigned char *>(a->workspace) + ws.partial_offset);
+    if (a->workspace == nullptr || a->tokens <= kPrefillWaveTokens) {
+        // 1 head and 2 waves a workgroup while the prompt is short (16
+        // workgroups a query block), 2 heads and 4 waves beyond.  N=211 f16:
+        // 9.2 us against 10.5, 700: 14.5 against 14.8, 1157: 24.5 against
+        // 22.2 (f32: 10.4 / 12.0, 16.7 / 17.7, 27.8 / 26.2).
+        const bool one = a->tokens <= kPrefillOneHeadTokens;
+        const dim3 grid(qblocks * kKvHeads * kGroup / (one ? 1 : 2)), threads(one ? 128 : 256);
+        if (one) {
+            if (f32) hipLaunchKernelGGL((prefill_wave_attention_kernel<true, 1, 2>), grid, threads, 0, st, p);
+            else hipLaunchKernelGGL((prefill_wave_attention_kernel<false, 1, 2>), grid, threads, 0, st, p);
+        } else {
+            if (f32) hipLaunchKernelGGL((prefill_wave_attention_kernel<true, 2, 4>), grid, threads, 0, st, p);
+            else hipLaunchKernelGGL((prefill_wave_attention_kernel<false, 2, 4>), grid, threads, 0, st, p);
+        }
+        return static_cast<int>(hipGetLastError());
     }
-    const unsigned grid = p.split ? prefill_pair_workgroups(qblocks) : qblocks * kKvHeads;
+    const PrefillWorkspace ws = prefill_workspace_layout(a->tokens);
+    p.counters = static_cast<uint32_t *>(a->workspace);
+    p.partials = reinterpret_cast<float *>(static_cast<unsigned char *>(a->workspace) + ws.partial_offset);
+    const unsigned grid = prefill_pair_workgroups(qblocks);
     if (f32) hipLaunchKernelGGL(prefill_attention_kernel<true>, dim3(grid), dim3(kWaves * 64), 0, st, p);
     else hipLaunchKernelGGL(prefill_attention_kernel<false>, dim3(grid), dim3(kWaves * 64), 0, st, p);
     return static_cast<int>(hipGetLastError());

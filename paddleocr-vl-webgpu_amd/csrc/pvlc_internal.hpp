@@ -201,7 +201,9 @@ int launch_linear_projection_f16(const float *input, const uint16_t *weight, con
 // then (otherwise the part that arrives last merges).  Running the heavy part
 // first lets the second workgroup find it complete and merge it without
 // storing its own part: config 4 at N=4096, 99.8-100.8 -> 96.6-97.3 us mean
-// per call.  Used when the longest block is longer than kPrefillSplitSteps.  A pair whose light workgroup
+// per call.  The workspace is asked for when the longest block is longer than
+// kPrefillSplitSteps and used by the prompts that launch_prefill gives to this
+// schedule.  A pair whose light workgroup
 // would take fewer than kPrefillSplitMin heavy steps at an even split is not
 // split (the light block and the heavy block run whole on the two
 // workgroups): a second segment costs its workgroup a query load, a pipeline
