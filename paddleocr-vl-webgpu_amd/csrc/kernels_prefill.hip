@@ -96,11 +96,17 @@ __device__ inline uint32_t cache_block(const PrefillParams &p, uint32_t tile, bo
 }
 
 // Kernel 1: one workgroup per 16-token cache block, both key heads.  Every
-// thread rotates two 8-dim key chunks (item = head, chunk, token; 16
-// consecutive threads fill one 256-byte run of the key slab) and writes one
-// 32-byte value row of the slab (head, dim: 16 tokens) after a transpose of
-// the block's value rows through LDS, so every cache store is a full 16-byte
-// vector and each 32-byte sector is written once.  With a query scratch the
+// thread rotates one pair of 8-dim key chunks, c and c + 8, which are each
+// other's rotary partners (item = head, chunk pair, token; 16 consecutive
+// threads fill one 256-byte run of the key slab), and writes one 32-byte value
+// row of the slab (head, dim: 16 tokens) after a transpose of the block's
+// value rows through LDS, so every cache store is a full 16-byte vector and
+// each 32-byte sector is written once.  It is bound by its chain of dependent
+// memory rounds, so there are three: positions, block id, keys and values;
+// cos and sin; the stores (the optional arrays are read through a stand-in
+// when not given, so no load waits behind a branch).  One chunk at a time,
+// positions read behind a branch for each, it took five: whole prefill calls
+// 25.7 -> 24.0 us at 1157 tokens, 84.6 -> 83.8 at 4096.  With a query scratch the
 // workgroup also writes the rotated queries of its tokens (the attention
 // kernel rotates its own query fragments, so the scratch is only an output for
 // callers that want it).
@@ -122,52 +128,85 @@ __global__ __launch_bounds__(kAppendThreads) void prefill_rope_append_kernel(Pre
     const uint32_t ntok = min(p.tokens - t0, kBlockTokens);
     __shared__ uint16_t sv[kBlockTokens][kRowElems + 8];  // value rows, padded against bank conflicts
 
-    // value rows of the block: 16 tokens x 256 fp16, two 16-byte pieces per
-    // thread, loaded now and staged into LDS after the key loads are issued
-    u16x8_t vrow[2];
+    const float *stand_in = F32IO ? p.value32 : reinterpret_cast<const float *>(p.value);
+    // item: head hh, chunk pair (c, c + 8), token t (the last one again past
+    // the end of the sequence, not stored)
+    const int tt = i & 15, c = (i >> 4) & 7, hh = i >> 7;
+    const uint32_t t = t0 + min(static_cast<uint32_t>(tt), ntok - 1);
+    const int32_t pos_raw = (p.positions ? p.positions : reinterpret_cast<const int32_t *>(stand_in))[t];
+    const int32_t id_raw = load_const(p.block_table ? p.block_table : reinterpret_cast<const int32_t *>(stand_in), b);
+    typedef std::conditional_t<F32IO, float4_t, half8_t> Raw;
+    constexpr int kRawLoads = F32IO ? 2 : 1, kRawElems = F32IO ? 4 : 8;
+    Raw key[2][kRawLoads], val[2][kRawLoads];
+    const size_t koff = (static_cast<size_t>(t) * kKvHeads + hh) * kHeadDim + c * 8;
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
+        // value rows of the block: 16 tokens x 256, two 8-element pieces per thread
         const int k = i + r * kAppendThreads;
-        const uint32_t t = t0 + min(static_cast<uint32_t>(k >> 5), ntok - 1);
-        if constexpr (F32IO)
-            vrow[r] = __builtin_bit_cast(u16x8_t, round_chunk(p.value32 + static_cast<size_t>(t) * kRowElems + (k & 31) * 8));
-        else
-            vrow[r] = *reinterpret_cast<const u16x8_t *>(p.value + static_cast<size_t>(t) * kRowElems + (k & 31) * 8);
-    }
-
-    bool ok;
-    const uint32_t blk = cache_block(p, b, &ok);
-    if (!ok && i == 0 && p.error_word) atomicOr(p.error_word, 2u);
-    // keys: item (head, chunk, token), 16 consecutive threads per 256-byte run
+        const size_t voff = static_cast<size_t>(t0 + min(static_cast<uint32_t>(k >> 5), ntok - 1)) * kRowElems + (k & 31) * 8;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int k = i + r * kAppendThreads;
-        const int tt = k & 15, c = (k >> 4) & 15, hh = k >> 8;
-        if (static_cast<uint32_t>(tt) < ntok) {
-            const uint32_t t = t0 + tt;
-            bool rope;
-            const int pos = rope_position(p, t, &rope);
-            if (!rope && p.rope_cos != nullptr && c == 0 && hh == 0 && p.error_word) atomicOr(p.error_word, 4u);
-            const size_t koff = (static_cast<size_t>(t) * kKvHeads + hh) * kHeadDim;
-            half8_t kv;
+        for (int f = 0; f < kRawLoads; ++f) {
             if constexpr (F32IO) {
-                kv = rope ? rotate_chunk(p.key32 + koff, c * 8, p.rope_cos + static_cast<size_t>(pos) * 64,
-                                         p.rope_sin + static_cast<size_t>(pos) * 64)
-                          : round_chunk(p.key32 + koff + c * 8);
+                key[r][f] = *reinterpret_cast<const Raw *>(p.key32 + koff + r * 64 + f * kRawElems);
+                val[r][f] = *reinterpret_cast<const Raw *>(p.value32 + voff + f * kRawElems);
             } else {
-                const uint16_t *krow = p.key + koff;
-                kv = rope ? rotate_chunk(krow, c * 8, p.rope_cos + static_cast<size_t>(pos) * 64,
-                                         p.rope_sin + static_cast<size_t>(pos) * 64)
-                          : *reinterpret_cast<const half8_t *>(krow + c * 8);
+                key[r][f] = *reinterpret_cast<const Raw *>(p.key + koff + r * 64);
+                val[r][f] = *reinterpret_cast<const Raw *>(p.value + voff);
             }
-            const size_t slab = (static_cast<size_t>(blk) * kKvHeads + hh) * kBlockHeadElems;
-            if (ok) *reinterpret_cast<half8_t *>(p.key_cache + slab + c * 128 + key_slot(tt) * 8) = kv;
         }
     }
+    const int pos = p.positions ? pos_raw : static_cast<int>(t);
+    const bool rope = p.rope_cos != nullptr && pos >= 0 && static_cast<uint32_t>(pos) < p.rope_rows;
+    float4_t cs[2], sn[2];
+    {
+        const float *cr = rope ? p.rope_cos + static_cast<size_t>(pos) * 64 + c * 8 : stand_in;
+        const float *sr = rope ? p.rope_sin + static_cast<size_t>(pos) * 64 + c * 8 : stand_in;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            cs[f] = *reinterpret_cast<const float4_t *>(cr + f * 4);
+            sn[f] = *reinterpret_cast<const float4_t *>(sr + f * 4);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load ahead of the arithmetic
+    const int32_t id = p.block_table ? id_raw : static_cast<int32_t>(b);
+    const bool ok = id >= 0 && static_cast<uint32_t>(id) < p.num_blocks;
+    const uint32_t blk = ok ? static_cast<uint32_t>(id) : 0u;
+    // keys, exactly as rotate_chunk rotates them
+    half8_t lo, hi;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float x = static_cast<float>(key[0][j / kRawElems][j % kRawElems]);
+        const float y = static_cast<float>(key[1][j / kRawElems][j % kRawElems]);
+        const float co = cs[j >> 2][j & 3], si = sn[j >> 2][j & 3];
+        lo[j] = to_h(rope ? x * co + (-y) * si : x);
+        hi[j] = to_h(rope ? y * co + x * si : y);
+    }
+    if constexpr (!F32IO) {
+        if (!rope) {  // as given, bit for bit
+            lo = key[0][0];
+            hi = key[1][0];
+        }
+    }
+    if (ok && static_cast<uint32_t>(tt) < ntok) {
+        uint16_t *dst = p.key_cache + (static_cast<size_t>(blk) * kKvHeads + hh) * kBlockHeadElems + c * 128 + key_slot(tt) * 8;
+        *reinterpret_cast<half8_t *>(dst) = lo;
+        *reinterpret_cast<half8_t *>(dst + 8 * 128) = hi;
+    }
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
         const int k = i + r * kAppendThreads;
-        *reinterpret_cast<u16x8_t *>(&sv[k >> 5][(k & 31) * 8]) = vrow[r];
+        half8_t v;
+        if constexpr (F32IO) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = to_h(val[r][j / kRawElems][j % kRawElems]);
+        } else {
+            v = val[r][0];
+        }
+        *reinterpret_cast<half8_t *>(&sv[k >> 5][(k & 31) * 8]) = v;
+    }
+    if (p.error_word) {
+        if (!ok && i == 0) atomicOr(p.error_word, 2u);
+        if (!rope && p.rope_cos != nullptr && c == 0 && hh == 0 && static_cast<uint32_t>(tt) < ntok) atomicOr(p.error_word, 4u);
     }
     __syncthreads();
     if (ok) {
