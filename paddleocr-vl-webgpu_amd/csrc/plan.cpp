@@ -10,6 +10,11 @@
 #include <limits>
 #include <string>
 
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+#define PVLC_HOST_F16C 1
+#include <immintrin.h>
+#endif
+
 #include "pvlc_internal.hpp"
 
 namespace pvlc {
@@ -41,12 +46,27 @@ PlanError require_len(size_t actual, uint64_t expected) {
     return none();
 }
 
+// Whether any value's magnitude bits are at least `bits` (0x7f800000: infinite
+// or NaN).  Whole runs are reduced before the test, so the loop vectorises.
+bool any_magnitude_from(const float *values, size_t n, uint32_t bits) {
+    constexpr size_t kRun = 2048;
+    for (size_t i = 0; i < n; i += kRun) {
+        const size_t end = n - i < kRun ? n : i + kRun;
+        uint32_t any = 0;
+        for (size_t j = i; j < end; ++j) {
+            uint32_t x;
+            std::memcpy(&x, values + j, 4);
+            any |= (x & 0x7fffffffu) >= bits ? 1u : 0u;
+        }
+        if (any) return true;
+    }
+    return false;
+}
+
 // require_finite, lib.rs:5261-5269
 PlanError require_finite(const float *values, size_t n) {
-    for (size_t i = 0; i < n; ++i) {
-        if (!std::isfinite(values[i]))
-            return err(PVLC_HIP_INV_NON_FINITE_INPUT, "floating input contains NaN or infinity");
-    }
+    if (any_magnitude_from(values, n, 0x7f800000u))
+        return err(PVLC_HIP_INV_NON_FINITE_INPUT, "floating input contains NaN or infinity");
     return none();
 }
 
@@ -288,11 +308,80 @@ float f16_to_f32(uint16_t bits) {
 }
 
 bool fp16_representable(const float *values, size_t n) {
-    for (size_t i = 0; i < n; ++i) {
-        if (!(std::fabs(values[i]) < 65520.0f)) return false;
-    }
-    return true;
+    return !any_magnitude_from(values, n, 0x477ff000u);  // 65520.0f and above, infinities, NaN
 }
+
+namespace {
+
+void block_slabs_scalar(const float *rows, uint32_t tokens, uint16_t *key_slab, uint16_t *value_slab) {
+    uint16_t *slab = key_slab ? key_slab : value_slab;
+    std::memset(slab, 0, sizeof(uint16_t) * kKvHeads * kBlockHeadElems);
+    for (uint32_t t = 0; t < tokens; ++t)
+        for (uint32_t h = 0; h < kKvHeads; ++h)
+            for (uint32_t d = 0; d < kHeadDim; ++d)
+                slab[key_slab ? key_blocked_index(t, h, d) : value_blocked_index(t, h, d)] =
+                    f32_to_f16_rne(rows[(static_cast<size_t>(t) * kKvHeads + h) * kHeadDim + d]);
+}
+
+#if defined(PVLC_HOST_F16C)
+// The same with the CPU's conversion instruction (round to nearest even; NaNs
+// quieted with their leading payload bits, as f32_to_f16_rne does) and 8 x 8
+// transposes of the values.
+__attribute__((target("avx,f16c"))) void block_slabs_f16c(const float *rows, uint32_t tokens, uint16_t *key_slab,
+                                                          uint16_t *value_slab) {
+    for (uint32_t h = 0; h < kKvHeads; ++h) {
+        for (uint32_t c = 0; c < kHeadDim / 8; ++c) {
+            __m128i v[kBlockTokens];
+            for (uint32_t t = 0; t < kBlockTokens; ++t)
+                v[t] = t < tokens ? _mm256_cvtps_ph(_mm256_loadu_ps(rows + (static_cast<size_t>(t) * kKvHeads + h) * kHeadDim + c * 8),
+                                                    _MM_FROUND_TO_NEAREST_INT)
+                                  : _mm_setzero_si128();
+            if (key_slab) {
+                uint16_t *dst = key_slab + h * kBlockHeadElems + c * (kBlockTokens * 8);
+                for (uint32_t t = 0; t < kBlockTokens; ++t)
+                    _mm_storeu_si128(reinterpret_cast<__m128i *>(dst + key_slot(static_cast<int>(t)) * 8), v[t]);
+                continue;
+            }
+            uint16_t *dst = value_slab + h * kBlockHeadElems + c * (8 * kBlockTokens);
+            for (uint32_t half = 0; half < 2; ++half) {
+                const __m128i *r = v + half * 8;
+                __m128i a[8], b[8];
+                for (int i = 0; i < 4; ++i) {  // pairs of tokens 2 i, 2 i + 1
+                    a[i] = _mm_unpacklo_epi16(r[2 * i], r[2 * i + 1]);
+                    a[i + 4] = _mm_unpackhi_epi16(r[2 * i], r[2 * i + 1]);
+                }
+                for (int i = 0; i < 2; ++i) {  // fours of tokens, dims 0-1, 2-3 | 4-5, 6-7
+                    b[4 * i] = _mm_unpacklo_epi32(a[4 * i], a[4 * i + 1]);
+                    b[4 * i + 1] = _mm_unpackhi_epi32(a[4 * i], a[4 * i + 1]);
+                    b[4 * i + 2] = _mm_unpacklo_epi32(a[4 * i + 2], a[4 * i + 3]);
+                    b[4 * i + 3] = _mm_unpackhi_epi32(a[4 * i + 2], a[4 * i + 3]);
+                }
+                for (int i = 0; i < 2; ++i)
+                    for (int j = 0; j < 2; ++j) {
+                        const int d = 4 * i + 2 * j;
+                        _mm_storeu_si128(reinterpret_cast<__m128i *>(dst + d * kBlockTokens + half * 8),
+                                         _mm_unpacklo_epi64(b[4 * i + j], b[4 * i + j + 2]));
+                        _mm_storeu_si128(reinterpret_cast<__m128i *>(dst + (d + 1) * kBlockTokens + half * 8),
+                                         _mm_unpackhi_epi64(b[4 * i + j], b[4 * i + j + 2]));
+                    }
+            }
+        }
+    }
+}
+#endif
+
+void block_slabs(const float *rows, uint32_t tokens, uint16_t *key_slab, uint16_t *value_slab) {
+#if defined(PVLC_HOST_F16C)
+    static const bool f16c = __builtin_cpu_supports("avx") && __builtin_cpu_supports("f16c");
+    if (f16c) return block_slabs_f16c(rows, tokens, key_slab, value_slab);
+#endif
+    block_slabs_scalar(rows, tokens, key_slab, value_slab);
+}
+
+}  // namespace
+
+void key_block_slabs(const float *rows, uint32_t tokens, uint16_t *slabs) { block_slabs(rows, tokens, slabs, nullptr); }
+void value_block_slabs(const float *rows, uint32_t tokens, uint16_t *slabs) { block_slabs(rows, tokens, nullptr, slabs); }
 
 size_t key_blocked_index(uint32_t token, uint32_t head, uint32_t dim) {
     const size_t block = token / kBlockTokens, t = token % kBlockTokens;

@@ -121,6 +121,11 @@ float f16_to_f32(uint16_t bits);
 // blocked device layout (contiguous blocks 0..ceil(tokens/16)-1).
 size_t key_blocked_index(uint32_t token, uint32_t head, uint32_t dim);
 size_t value_blocked_index(uint32_t token, uint32_t head, uint32_t dim);
+// The fp16 slabs (both heads) of one 16-token block from its compact f32 rows
+// [tokens][2][128], tokens of 1..16, rounded as f32_to_f16_rne rounds (the
+// other tokens are zero).
+void key_block_slabs(const float *rows, uint32_t tokens, uint16_t *slabs);
+void value_block_slabs(const float *rows, uint32_t tokens, uint16_t *slabs);
 
 // Kernel launchers (kernels_*.hip).  Return hipError_t as int.
 // The f32 operands of pvlc_hip_paged_decode_f32io (device pointers).

@@ -27,6 +27,20 @@
 
 using namespace pvlc;
 
+// What a session allocates: one device block (planes, step operands, attention
+// and workspace), one pinned block (a step's operands and results, then both
+// planes for the upload and the read-back) and its f32 rows.
+struct SessionBuffers {
+    char *device = nullptr;
+    size_t device_bytes = 0;
+    char *pinned = nullptr;
+    size_t pinned_bytes = 0;
+    // Host: the rows exactly as given, compact [capacity][2][128] f32 (the
+    // descriptor's planes, then each committed step's appended row).  The
+    // device planes hold these rounded to fp16; finish returns these.
+    std::vector<float> key_rows, value_rows;
+};
+
 struct pvlc_hip_runtime {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -40,6 +54,11 @@ struct pvlc_hip_runtime {
     std::mutex life_lock;
     uint32_t live_sessions = 0;
     bool destroy_requested = false;
+    // Buffers of a finished session, taken by the next one that they fit:
+    // allocating and freeing them took ~0.4 ms a session.  One set, of at most
+    // kMaxSpareBytes on the device and pinned each, freed with the runtime;
+    // used under the execution lock.
+    SessionBuffers spare;
 };
 
 struct pvlc_hip_kv_session {
@@ -50,6 +69,8 @@ struct pvlc_hip_kv_session {
     bool fail_next_after_submit = false;
     bool expire_next_wait = false;
     uint32_t num_blocks = 0;
+    SessionBuffers buffers;
+    // in buffers.device:
     uint16_t *key_cache = nullptr;    // blocked planes
     uint16_t *value_cache = nullptr;
     float *step_operands = nullptr;  // device: query | key | value (f32, rounded to fp16 by the kernel)
@@ -58,18 +79,18 @@ struct pvlc_hip_kv_session {
     // word with the attention
     float *attention = nullptr;
     void *workspace = nullptr;
-    float *host_staging = nullptr;  // pinned: operands in, attention and error word out
     size_t workspace_bytes = 0;
-    // Host: the rows exactly as given, compact [capacity][2][128] f32 (the
-    // descriptor's planes, then each committed step's appended row).  The
-    // device planes hold these rounded to fp16; finish returns these.
-    std::vector<float> key_rows, value_rows;
+    // in buffers.pinned:
+    float *host_staging = nullptr;  // a step's operands in, attention and error word out
+    uint16_t *host_planes = nullptr;  // key plane, value plane
 };
 
 namespace {
 
 constexpr size_t kQueryElems = kQueryHeads * kHeadDim;
 constexpr size_t kStepElems = kQueryElems + 2 * kRowElems;
+constexpr size_t kMaxSpareBytes = size_t{64} << 20;
+constexpr size_t align256(size_t v) { return (v + 255) & ~size_t{255}; }
 
 pvlc_hip_status hip_fail(hipError_t e, const char *what) {
     const int code = e == hipErrorOutOfMemory ? PVLC_HIP_OUT_OF_MEMORY : PVLC_HIP_OPERATION;
@@ -93,20 +114,22 @@ uint64_t now_ns() {
 constexpr uint64_t kDefaultWaitTimeoutNs = 30ull * 1000 * 1000 * 1000;
 
 // Wait for everything queued on the runtime's stream so far, at most the
-// runtime's timeout: an event recorded behind the work is polled, first
-// spinning, then sleeping 20 us between polls.  Returns hipSuccess, the HIP
+// runtime's timeout: an event recorded behind the work is polled, spinning for
+// the first 200 us (a step's work takes 30-50; a sleep of 20 us asked for ends
+// 70 us later), then sleeping 20 us between polls.  Returns hipSuccess, the HIP
 // error of the queue, or hipErrorNotReady when the deadline passed with the
 // work still pending.  `expire` reports the deadline as passed at the first
 // poll whatever the GPU's state (the tests' stand-in for a GPU that does not
 // finish, so that no GPU is made to hang).
 hipError_t wait_bounded(pvlc_hip_runtime *rt, bool expire) {
     if (hipError_t e = hipEventRecord(rt->done, rt->stream)) return e;
-    const uint64_t deadline = now_ns() + rt->wait_timeout_ns;
-    for (uint32_t polls = 0;; ++polls) {
+    const uint64_t begun = now_ns();
+    for (;;) {
         const hipError_t e = expire ? hipErrorNotReady : hipEventQuery(rt->done);
         if (e != hipErrorNotReady) return e;
-        if (expire || now_ns() >= deadline) return hipErrorNotReady;
-        if (polls >= 64) std::this_thread::sleep_for(std::chrono::microseconds(20));
+        const uint64_t waited = now_ns() - begun;
+        if (expire || waited >= rt->wait_timeout_ns) return hipErrorNotReady;
+        if (waited >= 200 * 1000) std::this_thread::sleep_for(std::chrono::microseconds(20));
     }
 }
 
@@ -123,29 +146,34 @@ pvlc_hip_status wait_or_fail(pvlc_hip_runtime *rt, bool expire, const char *what
     return PVLC_HIP_OK;
 }
 
-// Frees the session's buffers once the GPU work queued on the runtime has
-// completed (a bounded wait).  A session whose work does not complete within
-// the bound keeps its device buffers allocated (leaked) rather than freeing
-// memory a kernel may still access.
-void free_session_buffers(pvlc_hip_kv_session *s) {
-    if (!s) return;
-    if (s->runtime) {
-        (void)hipSetDevice(s->runtime->device);
-        if (wait_bounded(s->runtime, false) == hipErrorNotReady) return;  // pinned staging may still be written
-    }
-    (void)hipFree(s->key_cache);
-    (void)hipFree(s->value_cache);
-    (void)hipFree(s->step_operands);
-    (void)hipFree(s->attention);  // also holds the workspace
-    (void)hipHostFree(s->host_staging);
-    s->key_cache = s->value_cache = nullptr;
-    s->step_operands = s->attention = nullptr;
-    s->workspace = nullptr;
-    s->host_staging = nullptr;
+void free_buffers(SessionBuffers &b) {
+    (void)hipFree(b.device);
+    (void)hipHostFree(b.pinned);
+    b = SessionBuffers{};
+}
+
+// Gives the session's buffers back once the GPU work queued on the runtime
+// has completed (a bounded wait): to the runtime's spare set, or to the system
+// when that is taken, they are large, or the queue has failed.  A session
+// whose work does not complete within the bound keeps its buffers allocated
+// (leaked) rather than freeing memory a kernel or a copy may still access.
+void release_buffers(pvlc_hip_kv_session *s) {
+    pvlc_hip_runtime *rt = s->runtime;
+    (void)hipSetDevice(rt->device);
+    const hipError_t e = wait_bounded(rt, false);
+    if (e == hipErrorNotReady) return;
+    SessionBuffers &b = s->buffers;
+    if (e == hipSuccess && rt->spare.device == nullptr && b.device != nullptr && b.pinned != nullptr &&
+        b.device_bytes <= kMaxSpareBytes && b.pinned_bytes <= kMaxSpareBytes)
+        rt->spare = std::move(b);
+    else
+        free_buffers(b);
+    b = SessionBuffers{};
 }
 
 void destroy_runtime_now(pvlc_hip_runtime *rt) {
     (void)hipSetDevice(rt->device);
+    free_buffers(rt->spare);
     if (rt->done) (void)hipEventDestroy(rt->done);
     if (rt->stream) (void)hipStreamDestroy(rt->stream);
     delete rt;
@@ -161,7 +189,7 @@ void release_session(pvlc_hip_kv_session *s, bool lock_held) {
     {
         std::unique_lock<std::mutex> guard(rt->execution_lock, std::defer_lock);
         if (!lock_held) guard.lock();
-        free_session_buffers(s);
+        release_buffers(s);
     }
     delete s;
     bool last = false;
@@ -328,43 +356,53 @@ pvlc_hip_status create_session(pvlc_hip_runtime *rt, const pvlc_hip_kv_session_p
     };
     hipError_t e;
     if ((e = hipSetDevice(rt->device)) != hipSuccess) return cleanup(hip_fail(e, "hipSetDevice"));
-    if ((e = hipMalloc(&s->key_cache, plane_elems * 2)) != hipSuccess) return cleanup(hip_fail(e, "key cache"));
-    if ((e = hipMalloc(&s->value_cache, plane_elems * 2)) != hipSuccess) return cleanup(hip_fail(e, "value cache"));
-    if ((e = hipMalloc(&s->step_operands, kStepElems * 4)) != hipSuccess) return cleanup(hip_fail(e, "operands"));
-    if ((e = hipMalloc(&s->attention, kQueryElems * 4 + s->workspace_bytes)) != hipSuccess)
-        return cleanup(hip_fail(e, "attention and workspace"));
-    s->workspace = s->attention + kQueryElems;  // 8 KiB in: 256-byte aligned
-    if ((e = hipHostMalloc(reinterpret_cast<void **>(&s->host_staging), (kStepElems + kQueryElems + 1) * 4,
-                           hipHostMallocDefault)) != hipSuccess)
-        return cleanup(hip_fail(e, "pinned staging"));
+    // Device block: planes, step operands, attention (8 KiB, then the
+    // workspace: 256-byte aligned).  Pinned block: step staging, planes.
+    const size_t plane_bytes = align256(plane_elems * 2), operand_bytes = align256(kStepElems * 4);
+    const size_t device_bytes = 2 * plane_bytes + operand_bytes + kQueryElems * 4 + s->workspace_bytes;
+    const size_t staging_bytes = align256((kStepElems + kQueryElems + 1) * 4), pinned_bytes = staging_bytes + 2 * plane_elems * 2;
+    SessionBuffers &buf = s->buffers;
+    if (rt->spare.device_bytes >= device_bytes && rt->spare.pinned_bytes >= pinned_bytes) {
+        buf = std::move(rt->spare);
+        rt->spare = SessionBuffers{};
+    } else {
+        if ((e = hipMalloc(reinterpret_cast<void **>(&buf.device), device_bytes)) != hipSuccess)
+            return cleanup(hip_fail(e, "session device buffers"));
+        buf.device_bytes = device_bytes;
+        if ((e = hipHostMalloc(reinterpret_cast<void **>(&buf.pinned), pinned_bytes, hipHostMallocDefault)) != hipSuccess)
+            return cleanup(hip_fail(e, "pinned staging"));
+        buf.pinned_bytes = pinned_bytes;
+    }
+    s->key_cache = reinterpret_cast<uint16_t *>(buf.device);
+    s->value_cache = reinterpret_cast<uint16_t *>(buf.device + plane_bytes);
+    s->step_operands = reinterpret_cast<float *>(buf.device + 2 * plane_bytes);
+    s->attention = reinterpret_cast<float *>(buf.device + 2 * plane_bytes + operand_bytes);
+    s->workspace = s->attention + kQueryElems;
+    s->host_staging = reinterpret_cast<float *>(buf.pinned);
+    s->host_planes = reinterpret_cast<uint16_t *>(buf.pinned + staging_bytes);
 
     // Initial planes: keep the f32 rows, round to fp16 and scatter into the
-    // blocked layout on the host (rows past the capacity stay zero), then one
-    // copy per plane.
-    std::vector<uint16_t> kb, vb;
+    // blocked layout on the host (rows past the capacity are zero), one copy
+    // per plane, the first under way while the second is rounded.
     try {
         const size_t rows_elems = static_cast<size_t>(plan.cache_capacity) * kRowElems;
-        s->key_rows.assign(key_cache, key_cache + rows_elems);
-        s->value_rows.assign(value_cache, value_cache + rows_elems);
-        kb.assign(plane_elems, 0);
-        vb.assign(plane_elems, 0);
+        buf.key_rows.assign(key_cache, key_cache + rows_elems);
+        buf.value_rows.assign(value_cache, value_cache + rows_elems);
     } catch (const std::bad_alloc &) {
         return cleanup(fail(PVLC_HIP_OUT_OF_MEMORY, PVLC_HIP_INV_NONE, "host copy of the cache rows"));
     }
-    for (uint32_t t = 0; t < plan.cache_capacity; ++t) {
-        for (uint32_t h = 0; h < kKvHeads; ++h) {
-            for (uint32_t d = 0; d < kHeadDim; ++d) {
-                const size_t src = (static_cast<size_t>(t) * kKvHeads + h) * kHeadDim + d;
-                kb[key_blocked_index(t, h, d)] = f32_to_f16_rne(key_cache[src]);
-                vb[value_blocked_index(t, h, d)] = f32_to_f16_rne(value_cache[src]);
-            }
-        }
-    }
     hipStream_t st = rt->stream;
-    if ((e = hipMemcpyAsync(s->key_cache, kb.data(), plane_elems * 2, hipMemcpyHostToDevice, st)) != hipSuccess)
-        return cleanup(hip_fail(e, "key cache upload"));
-    if ((e = hipMemcpyAsync(s->value_cache, vb.data(), plane_elems * 2, hipMemcpyHostToDevice, st)) != hipSuccess)
-        return cleanup(hip_fail(e, "value cache upload"));
+    for (int plane = 0; plane < 2; ++plane) {
+        uint16_t *host = s->host_planes + plane * plane_elems;
+        const float *rows = plane ? buf.value_rows.data() : buf.key_rows.data();
+        for (uint32_t b = 0; b < s->num_blocks; ++b) {
+            const uint32_t t0 = b * kBlockTokens, left = plan.cache_capacity - t0;
+            const size_t at = static_cast<size_t>(t0) * kRowElems;
+            (plane ? value_block_slabs : key_block_slabs)(rows + at, left < kBlockTokens ? left : kBlockTokens, host + at);
+        }
+        if ((e = hipMemcpyAsync(plane ? s->value_cache : s->key_cache, host, plane_elems * 2, hipMemcpyHostToDevice, st)) != hipSuccess)
+            return cleanup(hip_fail(e, plane ? "value cache upload" : "key cache upload"));
+    }
     const int fe = launch_fill_u32(static_cast<uint32_t *>(s->workspace), s->workspace_bytes / 4, 0u, st);
     if (fe != 0) return cleanup(hip_fail(static_cast<hipError_t>(fe), "workspace init"));
     rt->counters.host_to_device_copies += 2;
@@ -431,8 +469,8 @@ pvlc_hip_status execute_step(pvlc_hip_kv_session *s, const pvlc_hip_kv_step_oper
                         std::to_string(device_error));
     std::memcpy(attention, result, kQueryElems * 4);
     const size_t row = static_cast<size_t>(s->cache_tokens) * kRowElems;
-    std::memcpy(s->key_rows.data() + row, step->appended_key, kRowElems * 4);
-    std::memcpy(s->value_rows.data() + row, step->appended_value, kRowElems * 4);
+    std::memcpy(s->buffers.key_rows.data() + row, step->appended_key, kRowElems * 4);
+    std::memcpy(s->buffers.value_rows.data() + row, step->appended_value, kRowElems * 4);
     if (exec) {
         exec->cache_tokens_before = s->cache_tokens;
         exec->cache_tokens_after = s->cache_tokens + 1;
@@ -451,19 +489,10 @@ pvlc_hip_status read_planes(pvlc_hip_kv_session *s, float *key_out, float *value
     pvlc_hip_runtime *rt = s->runtime;
     const size_t plane_elems = static_cast<size_t>(s->num_blocks) * kBlockTokens * kRowElems;
     HIP_TRY(hipSetDevice(rt->device), "hipSetDevice");
-    // Pinned staging keeps both copies asynchronous, so the one wait below
-    // (bounded) covers them.
-    uint16_t *staged = nullptr;
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&staged), plane_elems * 4, hipHostMallocDefault),
-            "finish staging");
-    struct Release {
-        uint16_t *p;
-        bool keep = false;  // the copies may still write into it
-        ~Release() {
-            if (!keep) (void)hipHostFree(p);
-        }
-    } release{staged};
-    uint16_t *kb = staged, *vb = staged + plane_elems;
+    // The session's pinned block keeps both copies asynchronous, so the one
+    // wait below (bounded) covers them; after an expired wait the session's
+    // release waits once more before it gives the block back.
+    uint16_t *kb = s->host_planes, *vb = s->host_planes + plane_elems;
     HIP_TRY(hipMemcpyAsync(kb, s->key_cache, plane_elems * 2, hipMemcpyDeviceToHost, rt->stream),
             "key cache readback");
     HIP_TRY(hipMemcpyAsync(vb, s->value_cache, plane_elems * 2, hipMemcpyDeviceToHost, rt->stream),
@@ -471,30 +500,33 @@ pvlc_hip_status read_planes(pvlc_hip_kv_session *s, float *key_out, float *value
     rt->counters.device_to_host_copies += 2;
     const bool expire = s->expire_next_wait;
     s->expire_next_wait = false;
-    if (pvlc_hip_status st = wait_or_fail(rt, expire, "decoder KV session finish")) {
-        // After a real time-out (or a failed queue) the copies may still write
-        // into the staging: it is kept (leaked) without waiting a second bound.
-        // After the tests' injected expiry one query of the event decides.
-        // The session's release makes the one remaining bounded wait.
-        release.keep = !expire || hipEventQuery(rt->done) != hipSuccess;
-        return st;
-    }
-    auto same = [](uint16_t device, float row) { return device == f32_to_f16_rne(row); };
-    for (uint32_t t = 0; t < s->plan.cache_capacity; ++t) {
-        for (uint32_t h = 0; h < kKvHeads; ++h) {
-            for (uint32_t d = 0; d < kHeadDim; ++d) {
-                const size_t src = (static_cast<size_t>(t) * kKvHeads + h) * kHeadDim + d;
-                if (!same(kb[key_blocked_index(t, h, d)], s->key_rows[src]) ||
-                    !same(vb[value_blocked_index(t, h, d)], s->value_rows[src]))
-                    return fail(PVLC_HIP_OPERATION, PVLC_HIP_INV_NONE,
-                                "decoder KV session finish: the device cache differs from the session's rows at row " +
-                                    std::to_string(t));
-            }
+    if (pvlc_hip_status st = wait_or_fail(rt, expire, "decoder KV session finish")) return st;
+    // Block by block: the slabs the rows round to, against the slabs read
+    // back; where they differ, the first row of the block that does.
+    const float *key_rows = s->buffers.key_rows.data(), *value_rows = s->buffers.value_rows.data();
+    constexpr size_t kBlockElems = static_cast<size_t>(kBlockTokens) * kRowElems;
+    uint16_t want[kBlockElems];
+    for (uint32_t b = 0; b < s->num_blocks; ++b) {
+        const uint32_t t0 = b * kBlockTokens, left = s->plan.cache_capacity - t0;
+        const uint32_t tokens = left < kBlockTokens ? left : kBlockTokens;
+        for (int plane = 0; plane < 2; ++plane) {
+            const uint16_t *got = (plane ? vb : kb) + b * kBlockElems;
+            (plane ? value_block_slabs : key_block_slabs)((plane ? value_rows : key_rows) + b * kBlockElems, tokens, want);
+            if (std::memcmp(got, want, sizeof(want)) == 0) continue;
+            for (uint32_t t = 0; t < tokens; ++t)
+                for (uint32_t h = 0; h < kKvHeads; ++h)
+                    for (uint32_t d = 0; d < kHeadDim; ++d) {
+                        const size_t at = plane ? value_blocked_index(t, h, d) : key_blocked_index(t, h, d);
+                        if (got[at] != want[at])
+                            return fail(PVLC_HIP_OPERATION, PVLC_HIP_INV_NONE,
+                                        "decoder KV session finish: the device cache differs from the session's rows at row " +
+                                            std::to_string(t0 + t));
+                    }
         }
     }
     const size_t rows_elems = static_cast<size_t>(s->plan.cache_capacity) * kRowElems;
-    std::memcpy(key_out, s->key_rows.data(), rows_elems * 4);
-    std::memcpy(value_out, s->value_rows.data(), rows_elems * 4);
+    std::memcpy(key_out, key_rows, rows_elems * 4);
+    std::memcpy(value_out, value_rows, rows_elems * 4);
     return PVLC_HIP_OK;
 }
 
