@@ -374,18 +374,19 @@ typedef struct pvlc_hip_paged_decode_args {
 } pvlc_hip_paged_decode_args;
 
 /* Partition size the automatic choice (partition_tokens = 0) plans with.  A
- * streaming launch (ragged cache_lens, or contexts beyond one round of
- * single-shot workgroups) may lengthen it on the device, to at most twice this
- * and at most 4096 tokens, so the items spread evenly over the compute units;
- * it records the partition it used in the workspace word after the error word
+ * streaming launch (partitions longer than 384 tokens, or ragged cache_lens
+ * with more than 512 workgroups of one (partition, kv head, sequence)) may
+ * lengthen it on the device, to at most twice this and at most 4096 tokens, so
+ * the items spread evenly over the compute units; it records the partition it
+ * used in the workspace word after the error word
  * (pvlc_hip_paged_decode_streaming_partition gives the same choice on the
- * host).  Ragged batches of more than 2048 sequences (more than the streaming
- * kernel numbers) run one workgroup per (partition, kv head, sequence) at
- * this partition instead, with the in-kernel merge. */
+ * host).  Other launches, and ragged batches of more than 2048 sequences (more
+ * than the streaming kernel numbers), run one workgroup per (partition, kv
+ * head, sequence) at this partition, with the in-kernel merge. */
 uint32_t pvlc_hip_paged_decode_partition(uint32_t num_seqs, uint32_t max_context);
-/* The partition an automatic launch over these ragged cache lengths (rows
- * cached before the append; host memory, num_seqs entries) settles on, on a
- * device of compute_units compute units: the planned partition P0 above, or
+/* The partition an automatic streaming launch over these ragged cache lengths
+ * (rows cached before the append; host memory, num_seqs entries) settles on, on
+ * a device of compute_units compute units: the planned partition P0 above, or
  * the candidate P0 + c*max(16, P0/4 rounded down to 16), c = 1..4, with the
  * least ceil(items / compute_units) * P, items counting (sequence, partition,
  * kv head) triples -- never longer than the 4096 tokens one streaming

@@ -279,10 +279,19 @@ pvlc_hip_status validate_decode_geometry(const pvlc_hip_paged_decode_args *a, ui
 pvlc_hip_status launch_decode_state(const pvlc_hip_paged_decode_args *a, uint32_t partition, uint32_t max_parts,
                                     const DecodeState &state, void *stream, uint32_t *launches_out,
                                     const DecodeOperands32 *f32) {
-    // Streaming regime: ragged lengths, or partitions longer than one chunk
-    // of the largest single-shot workgroup.
+    // Streaming regime: partitions longer than one chunk of the largest
+    // single-shot workgroup, or ragged lengths with more workgroups than two
+    // rounds of one per compute unit.  A smaller ragged launch takes one
+    // workgroup per (partition, kv head, sequence), those past the end of
+    // their sequence leaving at once: one launch instead of two, without the
+    // persistent kernel's pass over all lengths.  2 to 256 sequences of up to
+    // 128 to 6000 rows, every spread of lengths (all equal, 1:4, 1:16): 6-14 us
+    // against 11.5-17 (13 sequences up to 2010 rows 8.6 against 13.6; 256 up
+    // to 300, 512 workgroups, 14.3-17.9 against 16.1-19.6).
     const uint32_t part_tiles = (partition + kBlockTokens - 1) / kBlockTokens;
-    const bool streaming = (a->cache_lens != nullptr || part_tiles > kSingleShotTiles) && a->num_seqs <= kMaxRaggedSeqs;
+    const uint64_t workgroups = static_cast<uint64_t>(max_parts) * kKvHeads * a->num_seqs;
+    const bool streaming = a->num_seqs <= kMaxRaggedSeqs &&
+                           (part_tiles > kSingleShotTiles || (a->cache_lens != nullptr && workgroups > 2 * kTargetWorkgroups));
     const DecodeShape shape = decode_shape(partition, streaming);
     DecodeLaunch launch{a,
                         partition,
