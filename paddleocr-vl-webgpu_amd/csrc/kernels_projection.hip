@@ -419,44 +419,50 @@ __global__ __launch_bounds__(RW *KG * 64, MIN_WAVES) void projection_gemm_kernel
     }
 }
 
-// The tiles, largest first.
+// The tiles, by preference on equal cost.
 struct TileShape {
     uint32_t rows, cols;
 };
-constexpr TileShape kShapes[] = {{128, 192}, {128, 160}, {128, 128}, {128, 64}, {64, 64}, {32, 64}, {16, 64}, {16, 32}, {16, 16}};
+constexpr TileShape kShapes[] = {{128, 192}, {128, 160}, {128, 128}, {128, 64}, {64, 64}, {128, 96},
+                                  {64, 96},   {32, 64},   {16, 64},   {16, 32},  {16, 16}};
 constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
 
-// Order of the tiles: the column grouping with the smallest largest block
-// (the XCDs finish together), then the fewest operand bytes of that block (a
-// row of activations is twice a row of weights), and generations of columns
-// sized so that one generation is what an XCD runs at once.  *block receives
-// the tiles of the largest block.
+// Order of the tiles: the column grouping that gives the busiest compute unit
+// the fewest tiles (the XCDs finish together), then the fewest operand bytes
+// of an XCD's block (a row of activations is twice a row of weights), and
+// generations of columns sized so that one generation is what an XCD runs at
+// once.  *block receives the tiles of the largest block.  (The exact number of
+// tiles in the first place cost bytes for nothing: 1600 rows, o 29.6 us against
+// 26.7, down 37.1 against 34.7, four or eight column groups against one.)
 TileOrder tile_order(uint32_t row_tiles, uint32_t col_tiles, const TileShape &t, uint64_t *block) {
     TileOrder best{row_tiles, col_tiles, 1, 1};
-    uint64_t best_tiles = UINT64_MAX, best_bytes = UINT64_MAX;
+    uint64_t best_turns = UINT64_MAX, best_bytes = UINT64_MAX;
     for (uint32_t gc = 1; gc <= kXcds; gc *= 2) {
         const uint32_t gr = kXcds / gc;
         const uint64_t rb = (row_tiles + gr - 1) / gr, cb = (col_tiles + gc - 1) / gc;
-        const uint64_t bytes = rb * t.rows * 2 + cb * t.cols;
-        if (rb * cb < best_tiles || (rb * cb == best_tiles && bytes < best_bytes)) {
-            best_tiles = rb * cb;
+        const uint64_t turns = (rb * cb + kXcdUnits - 1) / kXcdUnits, bytes = rb * t.rows * 2 + cb * t.cols;
+        if (turns < best_turns || (turns == best_turns && bytes < best_bytes)) {
+            best_turns = turns;
             best_bytes = bytes;
             best.col_groups = gc;
+            *block = rb * cb;
         }
     }
     const uint32_t gr = kXcds / best.col_groups, rb = (row_tiles + gr - 1) / gr;
     best.gen = kXcdResident / rb > 0 ? kXcdResident / rb : 1;
-    *block = best_tiles;
     return best;
 }
 
 // The tile of a launch: the least clocks of the busiest compute unit per
 // 32-deep step, (tiles it runs) x max(matrix time, load time) with rows cols /
 // 32 clocks of MFMAs (hi and lo, 4096 FLOP per clock) and 2 rows + cols clocks
-// of loads (64 bytes per clock) a tile; the larger tile on ties.  The unit's
-// tiles are those of the largest XCD block over its 32 units.  Against every
-// tile timed at 16 to 4096 rows of the decoder's projections this picks the
-// fastest or one within 3% of it.
+// of loads (64 bytes per clock) a tile; on ties the earlier in the list (two
+// 64 x 64 tiles a unit overlap, one 128 x 96 does not: 300 rows of gate|up 17.5
+// against 19.1 us).  The unit's tiles are those of the largest XCD block over
+// its 32 units.  Against every tile timed at 16 to 4096 rows of the decoder's
+// projections this picks the fastest or one within 3% of it.  What the 96
+// column tiles save over the others: 400 rows, gate|up 23.3 -> 20.9 us; 900
+// rows, q|k|v 23.5 -> 20.8; 1157 rows, o 26.1 -> 24.0 and down 33.0 -> 30.4.
 int choose_tile(uint32_t rows, uint32_t k_width, uint32_t n_width, TileOrder *order, uint64_t *block) {
     int best = kShapeCount - 1;
     uint64_t best_cost = UINT64_MAX;
@@ -511,9 +517,11 @@ int launch_linear_projection_f16(const float *input, const uint16_t *weight, con
     case 2: PVLC_PROJECTION_LAUNCH(2, 4, 8, 1, 3, 3, 2); break;
     case 3: PVLC_PROJECTION_LAUNCH(2, 4, 4, 2, 3, 3, 2); break;
     case 4: PVLC_PROJECTION_LAUNCH(2, 2, 4, 2, 3, 3, 2); break;
-    case 5: PVLC_PROJECTION_LAUNCH(2, 1, 4, 4, 2, 4, 2); break;
-    case 6: PVLC_PROJECTION_LAUNCH(1, 1, 4, 4, 2, 4, 2); break;
-    case 7: PVLC_PROJECTION_LAUNCH(1, 1, 2, 8, 2, 4, 4); break;
+    case 5: PVLC_PROJECTION_LAUNCH(2, 4, 6, 2, 3, 3, 2); break;
+    case 6: PVLC_PROJECTION_LAUNCH(2, 2, 6, 2, 3, 3, 2); break;
+    case 7: PVLC_PROJECTION_LAUNCH(2, 1, 4, 4, 2, 4, 2); break;
+    case 8: PVLC_PROJECTION_LAUNCH(1, 1, 4, 4, 2, 4, 2); break;
+    case 9: PVLC_PROJECTION_LAUNCH(1, 1, 2, 8, 2, 4, 4); break;
     default: PVLC_PROJECTION_LAUNCH(1, 1, 1, 8, 2, 4, 4); break;
     }
 #undef PVLC_PROJECTION_LAUNCH

@@ -20,7 +20,9 @@ pytestmark = pytest.mark.gpu
                                       (64, 1056, 2560),   # 16 x 64: odd steps over 4 depth groups
                                       (128, 32, 2560),    # 32 x 64: three of four groups without a stage
                                       (211, 160, 2572),   # 64 x 64: two waves of rows, ragged rows
-                                      (385, 224, 2560),   # 128 x 64: two groups of four waves, one row in the last tile
+                                      (385, 224, 2560),   # 64 x 96: shifted last tile, one row in the last tile
+                                      (1601, 224, 1020),  # 128 x 64: two groups of four waves, one row in the last tile
+                                      (400, 96, 6140),    # 128 x 96: shifted last tile, odd steps
                                       (1157, 96, 2564),   # 128 x 128
                                       (2047, 160, 2556),  # 128 x 160: shifted last tile, ragged rows
                                       (2047, 352, 6136)]) # 128 x 192: shifted last tile, odd steps
