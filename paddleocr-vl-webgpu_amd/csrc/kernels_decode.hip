@@ -721,6 +721,33 @@ __device__ inline int64_t checked_cache_len(const DecodeParams &p, int64_t len) 
     return (len < 0 || len + 1 > capacity || len + 1 > span) ? -1 : len;
 }
 
+// x / d for integers 0 <= x, x + d < 2^19, 1 <= d <= 4096, x / d <= 2^19 / d:
+// the reciprocal (1 ulp) and the product move (x + 0.5) / d by less than
+// 2^19 / d 2^-22 < 0.25 / d, and it lies 0.5 / d or more from an integer.
+// Five instructions where a 32-bit division takes about thirty.
+__device__ inline uint32_t small_quotient(uint32_t x, uint32_t d) {
+    return static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(d)));
+}
+
+// Partitions of P tokens that the len + 1 rows of a sequence take (at most
+// kMaxMergeParts of 4096: checked_cache_len).
+__device__ inline uint32_t partitions_of(int64_t len, uint32_t P) {
+    return small_quotient(static_cast<uint32_t>(len) + P, P);
+}
+
+// Inclusive prefix sum over the lanes of a wave.
+__device__ inline uint32_t wave_inclusive_scan(uint32_t x) {
+#define PVLC_SCAN_STEP(CTRL, ROWS) x += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), CTRL, ROWS, 0xf, false))
+    PVLC_SCAN_STEP(0x111, 0xf);  // row_shr 1, 2, 4, 8 within each 16 lanes
+    PVLC_SCAN_STEP(0x112, 0xf);
+    PVLC_SCAN_STEP(0x114, 0xf);
+    PVLC_SCAN_STEP(0x118, 0xf);
+    PVLC_SCAN_STEP(0x142, 0xa);  // lane 15 of rows 0 and 2 to rows 1 and 3
+    PVLC_SCAN_STEP(0x143, 0xc);  // lane 31 to rows 2 and 3
+#undef PVLC_SCAN_STEP
+    return x;
+}
+
 // Grid (partition, kv head, sequence): sequences of one uniform length, or
 // ragged lengths when there are too many sequences for the ragged kernel.
 // The arguments the first key loads' addresses depend on come ahead of the
@@ -789,8 +816,8 @@ __device__ inline int workgroup_exclusive_scan(int v, int *sm_wave_sums, int *to
 }
 
 // Persistent grid for ragged lengths and long contexts: every workgroup
-// reads the cache lengths (and positions) once into LDS, numbers the (sequence, partition,
-// kv head) items that hold rows, and walks items blockIdx.x,
+// reads the cache lengths (and positions) once, into registers or LDS, numbers the
+// (sequence, partition, kv head) items that hold rows, and walks items blockIdx.x,
 // blockIdx.x + gridDim.x, ...  Sequences with fewer partitions launch no
 // empty workgroups, so every compute unit stays on real work, and the block
 // ids of the next item are loaded while the current one runs.
@@ -801,29 +828,15 @@ __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_ragged_kernel(Deco
     __shared__ int sm_len[kMaxRaggedSeqs];        // cache length, -1 if invalid
     __shared__ int sm_pos[kMaxRaggedSeqs];        // rotary position of the appended row
     __shared__ int sm_wave_sums[WAVES];
-    __shared__ int sm_counts[kPartitionChoices][WAVES];
+    __shared__ uint32_t sm_counts[kPartitionChoices][WAVES];
     const int n = static_cast<int>(num_seqs);
-    const int per = (n + kThreads - 1) / kThreads;
-    const int i0 = static_cast<int>(threadIdx.x) * per;
     // Validity is judged against the partition the host planned with.
     const int P0 = static_cast<int>(p.partition_tokens);
     static_assert(2 * PAIRS == 2, "wave_tile_ids holds 32 chunks of 2 tiles per wave");
     constexpr uint32_t kSpan = streaming_span(WAVES);
-    int counts[kPartitionChoices] = {};
-    for (int i = i0; i < min(i0 + per, n); ++i) {
-        const int64_t len =
-            checked_cache_len(p, p.cache_lens ? p.cache_lens[i] : static_cast<int64_t>(p.uniform_cache_len));
-        if (len < 0 && blockIdx.x == 0) atomicOr(p.error_word, 1u);
-        sm_len[i] = static_cast<int>(len);
-        sm_pos[i] = p.positions ? p.positions[i] : static_cast<int>(len);
-        if (p.partition_word) {
-#pragma unroll
-            for (int c = 0; c < kPartitionChoices; ++c) {
-                const int pc = static_cast<int>(streaming_partition_candidate(static_cast<uint32_t>(P0), c, kSpan));
-                counts[c] += (len < 0 || pc == 0) ? 0 : static_cast<int>((len + pc) / pc);
-            }
-        }
-    }
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint32_t units = max(1u, p.compute_units);
     // Automatic partition (choose_streaming_partition): item k runs on
     // workgroup k mod grid, and the grid fills every compute unit before it
     // doubles up, so item k lands on unit k mod units and a unit streams
@@ -831,50 +844,109 @@ __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_ragged_kernel(Deco
     // Every workgroup computes the same counts from the same lengths.  The
     // candidates stop at kSpan, the tokens covered by the block ids the
     // workgroup's waves hold (wave_tile_ids).
-    int P = P0;
-    if (p.partition_word) {
-        const int wave = threadIdx.x >> 6;
+    auto choose = [&](const uint32_t (&counts)[kPartitionChoices]) {  // partitions at each candidate
+        uint32_t turns[kPartitionChoices];
 #pragma unroll
         for (int c = 0; c < kPartitionChoices; ++c) {
-            int v = counts[c];
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o);
-            if ((threadIdx.x & 63) == 0) sm_counts[c][wave] = v;
+            // at most 2048 sequences x 64 partitions x 2 heads, 4096 units
+            turns[c] = __builtin_amdgcn_readfirstlane(small_quotient(counts[c] * kKvHeads + units - 1, units));
         }
-        __syncthreads();
-        const uint32_t units = max(1u, p.compute_units);
-        uint32_t items[kPartitionChoices] = {};
-        for (int c = 0; c < kPartitionChoices; ++c) {
-            for (int w = 0; w < WAVES; ++w) items[c] += static_cast<uint32_t>(sm_counts[c][w]);
-            items[c] *= kKvHeads;  // at most 2048 sequences x 64 partitions x 2 heads
-        }
-        P = static_cast<int>(choose_streaming_partition(items, static_cast<uint32_t>(P0), units, kSpan));
-        P = __builtin_amdgcn_readfirstlane(P);  // uniform: keep the item arithmetic scalar
+        const uint32_t best = best_streaming_partition(turns, static_cast<uint32_t>(P0), kSpan);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            p.partition_word[0] = static_cast<uint32_t>(P);
-            p.partition_word[1] = static_cast<uint32_t>(units);  // for inspection
+            p.partition_word[0] = best;
+            p.partition_word[1] = units;  // for inspection
         }
+        return static_cast<int>(__builtin_amdgcn_readfirstlane(best));  // uniform: keep the item arithmetic scalar
+    };
+    // Up to a wave's lanes of sequences every wave numbers them by itself, one
+    // per lane: no LDS and no barrier ahead of the first loads.  (Through LDS,
+    // with 64-bit divisions for the candidates, this prologue took 2.5 us more
+    // of every launch: 18 caches of 4096 rows 19.1 -> 16.6 us, 13 sequences up
+    // to 4096 rows 15.0 -> 12.6.  Several sequences per lane, for launches of
+    // up to 256, cost the small ones 0.8 us and won nothing.)
+    const bool in_lanes = n <= 64;  // uniform
+    int P = P0, total = 0;
+    int lane_len = -1, lane_pos = 0, lane_first = 0;
+    if (in_lanes) {
+        if (lane < n) {
+            lane_len = static_cast<int>(
+                checked_cache_len(p, p.cache_lens ? p.cache_lens[lane] : static_cast<int64_t>(p.uniform_cache_len)));
+            lane_pos = p.positions ? p.positions[lane] : lane_len;
+            if (lane_len < 0 && blockIdx.x == 0 && wave == 0) atomicOr(p.error_word, 1u);
+        }
+        auto parts_at = [&](uint32_t pc) { return lane_len < 0 || pc == 0 ? 0u : partitions_of(lane_len, pc); };
+        if (p.partition_word) {
+            uint32_t counts[kPartitionChoices];
+#pragma unroll
+            for (int c = 0; c < kPartitionChoices; ++c) {
+                const uint32_t x =
+                    wave_inclusive_scan(parts_at(streaming_partition_candidate(static_cast<uint32_t>(P0), c, kSpan)));
+                counts[c] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), 63));
+            }
+            P = choose(counts);
+        }
+        const uint32_t parts = parts_at(static_cast<uint32_t>(P)), through = wave_inclusive_scan(parts);
+        lane_first = static_cast<int>(through - parts);
+        total = __builtin_amdgcn_readlane(static_cast<int>(through), 63);
+    } else {
+        const int per = (n + kThreads - 1) / kThreads;
+        const int i0 = static_cast<int>(threadIdx.x) * per;
+        uint32_t counts[kPartitionChoices] = {};
+        for (int i = i0; i < min(i0 + per, n); ++i) {
+            const int64_t len =
+                checked_cache_len(p, p.cache_lens ? p.cache_lens[i] : static_cast<int64_t>(p.uniform_cache_len));
+            if (len < 0 && blockIdx.x == 0) atomicOr(p.error_word, 1u);
+            sm_len[i] = static_cast<int>(len);
+            sm_pos[i] = p.positions ? p.positions[i] : static_cast<int>(len);
+            if (p.partition_word) {
+#pragma unroll
+                for (int c = 0; c < kPartitionChoices; ++c) {
+                    const uint32_t pc = streaming_partition_candidate(static_cast<uint32_t>(P0), c, kSpan);
+                    counts[c] += len < 0 || pc == 0 ? 0u : partitions_of(len, pc);
+                }
+            }
+        }
+        if (p.partition_word) {
+#pragma unroll
+            for (int c = 0; c < kPartitionChoices; ++c) {
+                const uint32_t x = wave_inclusive_scan(counts[c]);
+                if (lane == 63) sm_counts[c][wave] = x;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < kPartitionChoices; ++c) {
+                counts[c] = 0;
+#pragma unroll
+                for (int w = 0; w < WAVES; ++w) counts[c] += sm_counts[c][w];
+            }
+            P = choose(counts);
+        }
+        int local = 0;
+        for (int i = i0; i < min(i0 + per, n); ++i) {
+            const int len = sm_len[i];  // written by this thread above
+            const int parts = len < 0 ? 0 : static_cast<int>(partitions_of(len, static_cast<uint32_t>(P)));
+            sm_first[i + 1] = parts;
+            local += parts;
+        }
+        int run = workgroup_exclusive_scan<kThreads>(local, sm_wave_sums, &total);
+        for (int i = i0; i < min(i0 + per, n); ++i) {
+            run += sm_first[i + 1];
+            sm_first[i + 1] = run;
+        }
+        if (threadIdx.x == 0) sm_first[0] = 0;
+        __syncthreads();
     }
-    int local = 0;
-    for (int i = i0; i < min(i0 + per, n); ++i) {
-        const int len = sm_len[i];  // written by this thread above
-        const int parts = len < 0 ? 0 : (len + P) / P;  // ceil((len + 1) / P)
-        sm_first[i + 1] = parts;
-        local += parts;
-    }
-    int total = 0;
-    int run = workgroup_exclusive_scan<kThreads>(local, sm_wave_sums, &total);
-    for (int i = i0; i < min(i0 + per, n); ++i) {
-        run += sm_first[i + 1];
-        sm_first[i + 1] = run;
-    }
-    if (threadIdx.x == 0) sm_first[0] = 0;
-    __syncthreads();
 
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    // Item k (per kv head) lies in the last sequence s with sm_first[s] <= k
+    // Item k (per kv head) lies in the last sequence s with first[s] <= k
     // (sequences without partitions share their successor's start).
-    auto locate = [&](int k, uint32_t *s_out, uint32_t *part_out) {
+    auto locate = [&](int k, uint32_t *s_out, uint32_t *part_out, int *len_out) {
+        if (in_lanes) {
+            const int s = __popcll(__ballot(lane < n && lane_first <= k)) - 1;  // the lanes 0 .. s
+            *s_out = static_cast<uint32_t>(s);
+            *part_out = static_cast<uint32_t>(k - __builtin_amdgcn_readlane(lane_first, s));
+            *len_out = __builtin_amdgcn_readlane(lane_len, s);
+            return;
+        }
         int lo = 0, hi = n - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -883,32 +955,36 @@ __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_ragged_kernel(Deco
         }
         *s_out = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(lo));
         *part_out = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(k - sm_first[lo]));
+        *len_out = __builtin_amdgcn_readfirstlane(sm_len[lo]);
     };
     const int items = total * static_cast<int>(kKvHeads);
     int item = blockIdx.x;
     if (item >= items) return;
     uint32_t s = 0, part = 0;
-    locate(item >> 1, &s, &part);
+    int len = 0;
+    locate(item >> 1, &s, &part, &len);
     bool bad = false;
     uint32_t ids = wave_tile_ids<WAVES, 2 * PAIRS>(p, s, static_cast<int>(part) * P,
-                                               min(static_cast<int>(part + 1) * P, sm_len[s] + 1), wave, &bad);
+                                               min(static_cast<int>(part + 1) * P, len + 1), wave, &bad);
     for (;;) {
         const int next = item + static_cast<int>(gridDim.x);
         uint32_t s_next = 0, part_next = 0, ids_next = 0;
+        int len_next = 0;
         bool bad_next = false;
         if (next < items) {
-            locate(next >> 1, &s_next, &part_next);
+            locate(next >> 1, &s_next, &part_next, &len_next);
             ids_next = wave_tile_ids<WAVES, 2 * PAIRS>(p, s_next, static_cast<int>(part_next) * P,
-                                                   min(static_cast<int>(part_next + 1) * P, sm_len[s_next] + 1), wave,
+                                                   min(static_cast<int>(part_next + 1) * P, len_next + 1), wave,
                                                    &bad_next);
         }
-        decode_item<WAVES, PAIRS, true, F32IO>(p, P, s, static_cast<uint32_t>(item & 1), part, sm_len[s], sm_pos[s],
-                                               ids, bad);
+        const int pos = in_lanes ? __builtin_amdgcn_readlane(lane_pos, static_cast<int>(s)) : sm_pos[s];
+        decode_item<WAVES, PAIRS, true, F32IO>(p, P, s, static_cast<uint32_t>(item & 1), part, len, pos, ids, bad);
         if (next >= items) break;
         __syncthreads();  // the next item reuses the workgroup's LDS
         item = next;
         s = s_next;
         part = part_next;
+        len = len_next;
         ids = ids_next;
         bad = bad_next;
     }
@@ -928,7 +1004,7 @@ __global__ __launch_bounds__(256) void paged_decode_merge_kernel(DecodeParams p)
     // The ragged kernel wrote the partition it used before this launch began.
     const int P = static_cast<int>(p.partition_word ? load_const(reinterpret_cast<const int32_t *>(p.partition_word), 0)
                                                     : p.partition_tokens);
-    const int num_parts = static_cast<int>((len + P) / P);
+    const int num_parts = static_cast<int>(partitions_of(len, static_cast<uint32_t>(P)));
     if (num_parts <= 1) return;
     const int e0 = threadIdx.x * 4;
     const int h = e0 >> 7;

@@ -64,26 +64,31 @@ constexpr uint32_t streaming_partition_candidate(uint32_t p0, int c, uint32_t sp
     const uint32_t pc = p0 + static_cast<uint32_t>(c) * (quarter > 16 ? quarter : 16);
     return pc <= span ? pc : 0;
 }
-// The candidate with the least ceil(items / units) * P (the first on ties),
-// where items[c] counts the (sequence, partition, kv head) items at candidate
-// c: item k runs on compute unit k mod units, so a unit streams
-// ceil(items / units) partitions one after the other.  p0 itself is a
-// candidate whenever p0 <= span, which the host's shape choice guarantees.
-constexpr uint32_t choose_streaming_partition(const uint32_t (&items)[kPartitionChoices], uint32_t p0,
-                                              uint32_t units, uint32_t span) {
-    const uint32_t u = units > 0 ? units : 1;
+// The candidate with the least turns * P (the first on ties), where turns[c] =
+// ceil(items / units) at candidate c and items counts its (sequence, partition,
+// kv head) items: item k runs on compute unit k mod units, so a unit streams
+// `turns` partitions one after the other.  p0 itself is a candidate whenever
+// p0 <= span, which the host's shape choice guarantees.
+constexpr uint32_t best_streaming_partition(const uint32_t (&turns)[kPartitionChoices], uint32_t p0, uint32_t span) {
     uint32_t best_p = p0;
     uint64_t best = ~0ull;
     for (int c = 0; c < kPartitionChoices; ++c) {
         const uint32_t pc = streaming_partition_candidate(p0, c, span);
         if (pc == 0) continue;
-        const uint64_t cost = static_cast<uint64_t>((items[c] + u - 1) / u) * pc;
+        const uint64_t cost = static_cast<uint64_t>(turns[c]) * pc;
         if (cost < best) {
             best = cost;
             best_p = pc;
         }
     }
     return best_p;
+}
+constexpr uint32_t choose_streaming_partition(const uint32_t (&items)[kPartitionChoices], uint32_t p0,
+                                              uint32_t units, uint32_t span) {
+    const uint32_t u = units > 0 ? units : 1;
+    uint32_t turns[kPartitionChoices] = {};
+    for (int c = 0; c < kPartitionChoices; ++c) turns[c] = (items[c] + u - 1) / u;
+    return best_streaming_partition(turns, p0, span);
 }
 
 // Status of a failed call: RuntimeErrorCode in bits 8..15, InvocationErrorCode
