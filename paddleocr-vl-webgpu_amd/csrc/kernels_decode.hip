@@ -821,7 +821,7 @@ __device__ inline int workgroup_exclusive_scan(int v, int *sm_wave_sums, int *to
 // blockIdx.x + gridDim.x, ...  Sequences with fewer partitions launch no
 // empty workgroups, so every compute unit stays on real work, and the block
 // ids of the next item are loaded while the current one runs.
-template <int WAVES, int PAIRS, bool F32IO>
+template <int WAVES, int PAIRS, bool F32IO, bool KEYS_FIRST>
 __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_ragged_kernel(DecodeParams p, uint32_t num_seqs) {
     constexpr int kThreads = WAVES * 64;
     __shared__ int sm_first[kMaxRaggedSeqs + 1];  // first item (per kv head) of each sequence
@@ -978,7 +978,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_ragged_kernel(Deco
                                                    &bad_next);
         }
         const int pos = in_lanes ? __builtin_amdgcn_readlane(lane_pos, static_cast<int>(s)) : sm_pos[s];
-        decode_item<WAVES, PAIRS, true, F32IO>(p, P, s, static_cast<uint32_t>(item & 1), part, len, pos, ids, bad);
+        decode_item<WAVES, PAIRS, true, F32IO, KEYS_FIRST>(p, P, s, static_cast<uint32_t>(item & 1), part, len, pos, ids, bad);
         if (next >= items) break;
         __syncthreads();  // the next item reuses the workgroup's LDS
         item = next;
@@ -1113,19 +1113,26 @@ int launch_paged_decode_kernels(const DecodeLaunch &launch, DecodeParams &p, hip
         // Persistent kernel storing partials, then the merge kernel: no
         // workgroup waits on a cross-workgroup hand-off.
         const uint64_t max_items = static_cast<uint64_t>(launch.max_parts) * kKvHeads * a.num_seqs;
-#define PVLC_RAGGED_LAUNCH(W, PR)                                                                                  \
+#define PVLC_RAGGED_LAUNCH(W, PR, KF)                                                                              \
     do {                                                                                                           \
         const uint32_t wgs = resident_workgroups(                                                                  \
-            reinterpret_cast<const void *>(&paged_decode_ragged_kernel<W, PR, F32IO>), (W) * 64, max_items,        \
+            reinterpret_cast<const void *>(&paged_decode_ragged_kernel<W, PR, F32IO, KF>), (W) * 64, max_items,    \
             &p.compute_units, &e);                                                                                 \
         if (e == 0) {                                                                                              \
-            hipLaunchKernelGGL((paged_decode_ragged_kernel<W, PR, F32IO>), dim3(wgs), dim3((W) * 64), 0, st, p,    \
-                               a.num_seqs);                                                                        \
+            hipLaunchKernelGGL((paged_decode_ragged_kernel<W, PR, F32IO, KF>), dim3(wgs), dim3((W) * 64), 0, st,   \
+                               p, a.num_seqs);                                                                     \
             hipLaunchKernelGGL(paged_decode_merge_kernel<F32IO>, dim3(kKvHeads, a.num_seqs), dim3(256), 0, st, p); \
         }                                                                                                          \
     } while (0)
-        if (launch.waves == 4) PVLC_RAGGED_LAUNCH(4, 1);
-        else PVLC_RAGGED_LAUNCH(2, 1);
+        // An f32 launch that rotates the query reads its small operands first
+        // (decode_item): the f32 rotation is then done when the keys arrive.
+        // Keys first against them first, f32: 18 caches of 3000 rows 15.9 / 14.6
+        // us, 16 sequences of 1000 to 8192 rows 16.4 / 15.0, 256 of 1024 to 8192
+        // 178.6 / 176.8, 32 of 4096 each 27.5 / 27.7; fp16: 14.4 / 14.4, 14.7 /
+        // 14.8, 169.5 / 169.9.
+        if (launch.waves != 4) PVLC_RAGGED_LAUNCH(2, 1, true);
+        else if (F32IO && p.rotate_query) PVLC_RAGGED_LAUNCH(4, 1, !F32IO);
+        else PVLC_RAGGED_LAUNCH(4, 1, true);
 #undef PVLC_RAGGED_LAUNCH
         if (e != 0) return e;
         return static_cast<int>(hipGetLastError());
