@@ -56,7 +56,8 @@ struct pvlc_hip_runtime {
     bool destroy_requested = false;
     // Buffers of a finished session, taken by the next one that they fit:
     // allocating and freeing them took ~0.4 ms a session.  One set, of at most
-    // kMaxSpareBytes on the device and pinned each, freed with the runtime;
+    // kMaxSpareBytes on the device and pinned each, freed with the runtime or
+    // when a session finds it too small;
     // used under the execution lock.
     SessionBuffers spare;
 };
@@ -375,6 +376,7 @@ pvlc_hip_status create_session(pvlc_hip_runtime *rt, const pvlc_hip_kv_session_p
         buf = std::move(rt->spare);
         rt->spare = SessionBuffers{};
     } else {
+        free_buffers(rt->spare);  // too small: its memory is free for this session, and this session's set is kept instead
         if ((e = hipMalloc(reinterpret_cast<void **>(&buf.device), device_bytes)) != hipSuccess)
             return cleanup(hip_fail(e, "session device buffers"));
         buf.device_bytes = device_bytes;
