@@ -1,5 +1,6 @@
 // Causal prefill for gfx950: rotary + range append into the paged cache, then
-// MFMA flash attention over the cache.
+// MFMA flash attention over the cache; both in one kernel for short prompts
+// (prefill_short_kernel).
 //
 // Kernel 1 (one 16-token cache block per workgroup): rotates the 2 key heads
 // and writes them with the values into the blocked cache (the same rounding as the decode
@@ -1124,6 +1125,323 @@ __global__ __launch_bounds__(KG * 64, 2) void prefill_wave_attention_kernel(Pref
     }
 }
 
+// Prompts of at most kPrefillShortTokens in one launch: append and attention
+// together.  A workgroup takes one head of a 16-token query block, and wave w
+// its 32-key step w, so there is no loop.  Keys and values come from the
+// call's own rows, not from the cache that another workgroup is writing: each
+// wave rotates and rounds its keys in registers (the same arithmetic, hence
+// the same bits, as the append kernel), its values pass through LDS into P.V
+// operand order, and the first head of each group stores the query block's
+// own rows into the cache.
+//
+// What bounds it: latency (the launch; positions and rows; cos and sin; the
+// merge), and from three steps on the compute unit's load path: rows and angles
+// of a step are 32 KiB, in lines half used, for every head and later query
+// block again.  Two launches pay that once, and a launch gap.  us a call, one
+// launch / two (f16, then f32): 16 tokens 5.1 / 7.7, 5.4 / 7.8; 64 tokens 5.7 /
+// 7.5, 6.3 / 7.7; 96 tokens 6.5 / 7.6, 7.4 / 7.9; 128 tokens 7.3 / 7.6, 8.4 /
+// 8.0; 211 tokens 11.1 / 8.1, 13.0 / 9.0.
+constexpr uint32_t kPrefillShortTokens = 96;
+constexpr int kShortWaves = 4;  // the last one has no keys: with the one before it, it rotates the query
+static_assert(kPrefillShortTokens <= kShortWaves * 32, "a wave for each step");
+
+template <bool F32IO>
+__global__ __launch_bounds__(kShortWaves * 64, 2) void prefill_short_kernel(PrefillParams p) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int KG = kShortWaves;
+    const int n = static_cast<int>(p.tokens);
+    const int qblocks = (n + kQueryBlock - 1) / kQueryBlock;
+    const uint32_t g = blockIdx.x & 1u;
+    const int hs = static_cast<int>((blockIdx.x >> 1) % kGroup);
+    const int qb = qblocks - 1 - static_cast<int>((blockIdx.x >> 1) / kGroup);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int row = lane & 15, kg = lane >> 4;
+    const int t0 = qb * kQueryBlock, my_token = t0 + row;
+    const int steps = (qb + 2) >> 1, k0 = wave * 32;  // 32-key steps of the block; first key of this wave's
+    const bool live = wave < steps;                   // uniform
+    const int h0 = static_cast<int>(g) * kGroup + hs;
+
+    constexpr int kRow = kHeadDim + 4;  // padded against bank conflicts
+    __shared__ float sm_m[KG][16], sm_l[KG][16];
+    __shared__ __align__(16) half8_t sm_q[4 * 64];  // [kb][lane]
+    // a wave's values [32 tokens][kRow fp16], then (behind a barrier) its O [16][kRow f32]
+    __shared__ __align__(16) float sm_o[KG][16][kRow];
+    uint32_t *sm_v = reinterpret_cast<uint32_t *>(&sm_o[wave][0][0]);
+
+    typedef std::conditional_t<F32IO, float4_t, half8_t> Raw;
+    constexpr int kRawLoads = F32IO ? 2 : 1, kRawElems = F32IO ? 4 : 8;
+    auto raw_load = [&](const float *src32, const uint16_t *src, size_t at, Raw (&dst)[kRawLoads]) {
+#pragma unroll
+        for (int f = 0; f < kRawLoads; ++f) {
+            if constexpr (F32IO) dst[f] = *reinterpret_cast<const Raw *>(src32 + at + f * kRawElems);
+            else dst[f] = *reinterpret_cast<const Raw *>(src + at);
+        }
+    };
+    // Lane (row, kg) holds, for score MFMA h, the key in slot h * 8 + row % 8
+    // of tile row / 8 of the step, dims kb * 32 + kg * 8 .. +8 (as load_k of
+    // prefill_wave_attention_kernel); tokens past the end repeat the last one.
+    // Optional arrays are read through the query when not given, so that no
+    // load waits behind a branch.
+    const int32_t *stand_in = F32IO ? reinterpret_cast<const int32_t *>(p.query32) : reinterpret_cast<const int32_t *>(p.query);
+    const int key_tile = 2 * wave + (row >> 3);
+    int kt[2], kpos_raw[2];
+    const int tq = min(my_token, n - 1);
+    const int qpos_raw = (p.positions ? p.positions : stand_in)[tq];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        kt[h] = min(key_tile * 16 + key_slot(h * 8 + (row & 7)), n - 1);
+        kpos_raw[h] = (p.positions ? p.positions : stand_in)[kt[h]];
+    }
+    const int32_t id_raw = load_const(p.block_table ? p.block_table : stand_in, static_cast<uint32_t>(qb));
+    const float *stand_in32 = reinterpret_cast<const float *>(stand_in);
+    auto rope_at = [&](int raw, int t, bool *rope) {
+        const int pos = p.positions ? raw : t;
+        *rope = p.rope_cos != nullptr && pos >= 0 && static_cast<uint32_t>(pos) < p.rope_rows;
+        return static_cast<size_t>(pos) * 64;
+    };
+    auto rotate_pair = [&](const Raw (&a)[kRawLoads], const Raw (&b)[kRawLoads], const float4_t *cs, const float4_t *sn,
+                           bool rope, half8_t *lo, half8_t *hi) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float x = static_cast<float>(a[j / kRawElems][j % kRawElems]);
+            const float y = static_cast<float>(b[j / kRawElems][j % kRawElems]);
+            const float co = cs[j >> 2][j & 3], si = sn[j >> 2][j & 3];
+            (*lo)[j] = to_h(rope ? x * co + (-y) * si : x);
+            (*hi)[j] = to_h(rope ? y * co + x * si : y);
+        }
+        if constexpr (!F32IO) {
+            if (!rope) {  // as given, bit for bit
+                *lo = a[0];
+                *hi = b[0];
+            }
+        }
+    };
+    half8_t kf[2][4];
+    bool krope[2] = {true, true};
+    if (live) {
+        Raw kr[2][4][kRawLoads], vr[8][kRawLoads];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb)
+                raw_load(p.key32, p.key, (static_cast<size_t>(kt[h]) * kKvHeads + g) * kHeadDim + kb * 32 + kg * 8, kr[h][kb]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)  // value pieces: token j * 4 + kg of the step, 16 bytes `row` of its fp16 row
+            raw_load(p.value32, p.value, (static_cast<size_t>(min(k0 + j * 4 + kg, n - 1)) * kKvHeads + g) * kHeadDim + row * 8, vr[j]);
+        float4_t kc[2][2][2], ks[2][2][2];  // [h][dims hk * 32 + kg * 8 .. +8]
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const size_t at = rope_at(kpos_raw[h], kt[h], &krope[h]);
+            const float *cr = krope[h] ? p.rope_cos + at : stand_in32, *sr = krope[h] ? p.rope_sin + at : stand_in32;
+#pragma unroll
+            for (int hk = 0; hk < 2; ++hk)
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    kc[h][hk][f] = *reinterpret_cast<const float4_t *>(cr + hk * 32 + kg * 8 + f * 4);
+                    ks[h][hk][f] = *reinterpret_cast<const float4_t *>(sr + hk * 32 + kg * 8 + f * 4);
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every load ahead of the arithmetic
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            half8_t v;
+            if constexpr (F32IO) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = to_h(vr[j][e / kRawElems][e % kRawElems]);
+            } else {
+                v = vr[j][0];
+            }
+            const u32x4 w = __builtin_bit_cast(u32x4, v);
+            u32x2 *dst = reinterpret_cast<u32x2 *>(sm_v + (j * 4 + kg) * (kRow / 2) + row * 4);  // 8-byte aligned
+            dst[0] = u32x2{w[0], w[1]};
+            dst[1] = u32x2{w[2], w[3]};
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                rotate_pair(kr[h][kb], kr[h][kb + 2], kc[h][kb], ks[h][kb], krope[h], &kf[h][kb], &kf[h][kb + 2]);
+    }
+    // Query fragments (B operand: column = token t0 + row, dims kb * 32 + kg *
+    // 8 .. +8): the last two waves, most often without keys, take one rotary
+    // pair (kb, kb + 2) each.
+    if (wave >= KG - 2) {  // uniform
+        const int kb = wave - (KG - 2);
+        const size_t at = (static_cast<size_t>(tq) * kQueryHeads + h0) * kHeadDim + kb * 32 + kg * 8;
+        Raw a[kRawLoads], b[kRawLoads];
+        raw_load(p.query32, p.query, at, a);
+        raw_load(p.query32, p.query, at + 64, b);
+        bool rope;
+        const size_t tab = rope_at(qpos_raw, tq, &rope);
+        const float *cr = rope ? p.rope_cos + tab : stand_in32, *sr = rope ? p.rope_sin + tab : stand_in32;
+        float4_t cs[2], sn[2];
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            cs[f] = *reinterpret_cast<const float4_t *>(cr + kb * 32 + kg * 8 + f * 4);
+            sn[f] = *reinterpret_cast<const float4_t *>(sr + kb * 32 + kg * 8 + f * 4);
+        }
+        half8_t lo, hi;
+        rotate_pair(a, b, cs, sn, rope, &lo, &hi);
+        sm_q[kb * 64 + lane] = lo;
+        sm_q[(kb + 2) * 64 + lane] = hi;
+    }
+    __syncthreads();
+
+    float4_t o[9];  // dims (c / 2) * 32 + 2 * row + c % 2 of 8 column tiles, then the row sums
+#pragma unroll
+    for (int c = 0; c < 9; ++c) o[c] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const float scale = p.scale_log2;
+    float m_run = -INFINITY;
+    if (live) {
+        float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            const half8_t qf = sm_q[kb * 64 + lane];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[h][kb], qf, acc[h], 0, 0, 0);
+        }
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int key = k0 + kg * 8 + e;
+            x[e] = key <= my_token && key < n ? acc[e >> 2][e & 3] : -INFINITY;
+            m_run = fmaxf(m_run, x[e]);
+        }
+        {  // over the 4 lanes of a column
+            u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(m_run), __float_as_uint(m_run), false, false));
+            m_run = fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+            v = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(m_run), __float_as_uint(m_run), false, false));
+            m_run = fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+        }
+        const float ms = m_run == -INFINITY ? 0.f : m_run * scale;
+        half8_t hi, lo, ones;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float pf = __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], scale, -ms));
+            hi[e] = to_h(pf);
+            lo[e] = F32IO ? to_h(pf - static_cast<float>(hi[e])) : static_cast<_Float16>(0.0f);
+            ones[e] = static_cast<_Float16>(1.0f);
+        }
+        // The query block's own rows into the cache, from the workgroup of the
+        // group's first head: keys as they lie in kf, values as in vf below.
+        const bool writer = hs == 0 && wave == steps - 1;  // uniform
+        const int32_t id = p.block_table ? id_raw : static_cast<int32_t>(qb);
+        const bool ok = id >= 0 && static_cast<uint32_t>(id) < p.num_blocks;
+        const size_t slab = (static_cast<size_t>(ok ? id : 0) * kKvHeads + g) * kBlockHeadElems;
+        if (writer && key_tile == qb) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int slot = h * 8 + (row & 7);
+                if (qb * 16 + key_slot(slot) >= n) continue;
+                if (p.error_word && kg == 0 && !krope[h] && p.rope_cos != nullptr) atomicOr(p.error_word, 4u);
+                if (!ok) continue;
+#pragma unroll
+                for (int kb = 0; kb < 4; ++kb)
+                    *reinterpret_cast<half8_t *>(p.key_cache + slab + (kb * 4 + kg) * 128 + slot * 8) = kf[h][kb];
+            }
+        }
+        if (writer && !ok && lane == 0 && p.error_word) atomicOr(p.error_word, 2u);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            // keys kg * 8 .. +8 of dims c * 32 + 2 * row and the next: 32 banks
+            // apart over kg, one dword each over row
+            uint32_t d[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) d[e] = sm_v[(kg * 8 + e) * (kRow / 2) + c * 16 + row];
+            u32x4 even, odd;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                even[e] = (d[2 * e] & 0xffffu) | (d[2 * e + 1] << 16);
+                odd[e] = (d[2 * e] >> 16) | (d[2 * e + 1] & 0xffff0000u);
+            }
+            const half8_t vf[2] = {__builtin_bit_cast(half8_t, even), __builtin_bit_cast(half8_t, odd)};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                o[2 * c + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, vf[i], o[2 * c + i], 0, 0, 0);
+                if constexpr (F32IO) o[2 * c + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, vf[i], o[2 * c + i], 0, 0, 0);
+            }
+            if (writer && ok && 2 * wave + (kg >> 1) == qb) {
+                const int left = n - (qb * 16 + (kg & 1) * 8);  // tokens of this half
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    uint16_t *dst = p.value_cache + slab + (c * 32 + 2 * row + i) * 16 + (kg & 1) * 8;
+                    if (left >= 8) {
+                        *reinterpret_cast<half8_t *>(dst) = vf[i];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            if (e < left) dst[e] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(vf[i][e]));
+                    }
+                }
+            }
+        }
+        o[8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, ones, o[8], 0, 0, 0);
+        if constexpr (F32IO) o[8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, ones, o[8], 0, 0, 0);
+    }
+
+    // Merge, as in prefill_wave_attention_kernel (waves without a step are left out).
+    if (kg == 0) sm_m[wave][row] = m_run;
+    __syncthreads();  // and every wave has read its values
+    if (live) {
+        float m = sm_m[0][row];
+        for (int w = 1; w < steps; ++w) m = fmaxf(m, sm_m[w][row]);
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m) * scale);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float a = __shfl(alpha, kg * 4 + r);
+            float *dst = sm_o[wave][kg * 4 + r] + 2 * row;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) dst[(c >> 1) * 32 + (c & 1)] = o[c][r] * a;
+            if (row == 0) sm_l[wave][kg * 4 + r] = o[8][r] * a;
+        }
+    }
+    __syncthreads();
+    constexpr int kChunks = kQueryBlock * kHeadDim / 4;  // of 4 outputs
+    static_assert(kChunks % (KG * 64) == 0, "every thread stores the same number of chunks");
+#pragma unroll
+    for (int j = 0; j < kChunks / (KG * 64); ++j) {
+        const int q = j * (KG * 64) + static_cast<int>(threadIdx.x), r = q / (kHeadDim / 4), d0 = q % (kHeadDim / 4) * 4, t = t0 + r;
+        float l = 0.f;
+        float4_t v = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int w = 0; w < steps; ++w) {
+            l += sm_l[w][r];
+            v += *reinterpret_cast<const float4_t *>(&sm_o[w][r][d0]);
+        }
+        if (t < n) {
+            const float inv = 1.0f / l;
+            const size_t off = (static_cast<size_t>(t) * kQueryHeads + h0) * kHeadDim + d0;
+            if constexpr (F32IO) {
+                *reinterpret_cast<float4_t *>(p.out32 + off) = v * inv;
+            } else {
+                typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+                half4 h;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) h[e] = to_h(v[e] * inv);
+                *reinterpret_cast<half4 *>(p.out + off) = h;
+            }
+        }
+    }
+}
+
+// Whether the call's key and value rows lie apart from everything the
+// one-launch form writes while other workgroups still read them.
+bool rows_apart(const PrefillParams &p, bool f32) {
+    const size_t bytes = f32 ? 4 : 2, rows = p.tokens * size_t{kRowElems} * bytes;
+    const size_t plane = static_cast<size_t>(p.num_blocks) * kKvHeads * kBlockHeadElems * 2;
+    auto apart = [](const void *a, size_t an, const void *b, size_t bn) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+        return x + an <= y || y + bn <= x;
+    };
+    const void *out = f32 ? static_cast<const void *>(p.out32) : p.out;
+    for (const void *in : {f32 ? static_cast<const void *>(p.key32) : p.key, f32 ? static_cast<const void *>(p.value32) : p.value})
+        if (!apart(in, rows, out, rows / kKvHeads * kQueryHeads) || !apart(in, rows, p.key_cache, plane) ||
+            !apart(in, rows, p.value_cache, plane))
+            return false;
+    return true;
+}
+
 }  // namespace
 
 int launch_prefill(const pvlc_hip_paged_prefill_args *a, void *stream, const PrefillOperands32 *f32) {
@@ -1151,6 +1469,12 @@ int launch_prefill(const pvlc_hip_paged_prefill_args *a, void *stream, const Pre
         p.out32 = f32->out;
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (a->tokens <= kPrefillShortTokens && a->query_scratch == nullptr && rows_apart(p, f32 != nullptr)) {
+        const dim3 grid((a->tokens + kQueryBlock - 1) / kQueryBlock * kQueryHeads), threads(kShortWaves * 64);
+        if (f32) hipLaunchKernelGGL(prefill_short_kernel<true>, grid, threads, 0, st, p);
+        else hipLaunchKernelGGL(prefill_short_kernel<false>, grid, threads, 0, st, p);
+        return static_cast<int>(hipGetLastError());
+    }
     const dim3 append_grid((a->tokens + kBlockTokens - 1) / kBlockTokens);
     if (f32) hipLaunchKernelGGL(prefill_rope_append_kernel<true>, append_grid, dim3(kAppendThreads), 0, st, p);
     else hipLaunchKernelGGL(prefill_rope_append_kernel<false>, append_grid, dim3(kAppendThreads), 0, st, p);
