@@ -11,7 +11,8 @@
 //
 // Kernel 2 (attention) has two forms, chosen in launch_prefill:
 //
-//  * prefill_wave_attention_kernel (prompts up to kPrefillWaveTokens, and any
+//  * prefill_wave_attention_kernel (prompts beyond kPrefillShortTokens or with
+//    a query scratch, up to kPrefillWaveTokens, and any
 //    length without a workspace): one workgroup per (16-token query block, 1
 //    or 2 heads), its waves taking the key steps in turn, each streaming its
 //    keys and values from L2 into registers with no barrier in the loop, and

@@ -1,5 +1,5 @@
-"""The prefill attention that spreads a query block's heads and keys over workgroups and waves (prompts up to 3072
-tokens, and any length without a workspace), around the edges it can go wrong at: query blocks and 32-key steps partly
+"""The prefill attention that spreads a query block's heads and keys over workgroups and waves (prompts of 97 to 3072
+tokens, any greater length without a workspace, and the one-launch form of up to 96 tokens), around the edges it can go wrong at: query blocks and 32-key steps partly
 filled, waves without a step, the switch of its one- and two-head forms, block ids reloaded after 32 steps a wave, and
 the first lengths of the pair schedule.  Every output row against a 64-bit softmax over the same fp16 operands, in both
 operand widths, through a permuted block table with spare blocks.
