@@ -97,6 +97,17 @@ __device__ inline uint32_t cache_block(const PrefillParams &p, uint32_t tile, bo
     return *ok ? static_cast<uint32_t>(b) : 0u;
 }
 
+// Mask of the values of keys key .. key + 7 that belong to a prompt of n tokens.
+// A partly filled last block keeps what the planes held in its other tokens:
+// their weights are 0, but 0 times a NaN or an infinity there is NaN.
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+__device__ inline u32x4_t value_keep(int key, int n) {
+    u32x4_t keep;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) keep[d] = key + 2 * d + 1 < n ? ~0u : key + 2 * d < n ? 0xffffu : 0u;
+    return keep;
+}
+
 // Kernel 1: one workgroup per 16-token cache block, both key heads.  Every
 // thread rotates one pair of 8-dim key chunks, c and c + 8, which are each
 // other's rotary partners (item = head, chunk pair, token; 16 consecutive
@@ -658,6 +669,19 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_kernel(Prefi
     // and are spilled around it.
     const int tail_lane = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
     for (; i < steps; ++i) {  // the last one to three steps
+        if (i + 1 == steps && last_part && t0 + kQueryBlock > n) {  // uniform: the block's tokens end inside a cache block
+            // V(i) has landed; its tokens past the prompt are zeroed in LDS
+            // (value_keep): one tile a round, half and dim by thread.
+            uint16_t *vl = (i & 1) != 0 ? sv1 : sv0;
+            const int half = wave >> 1, dim = (wave & 1) * 64 + tail_lane;
+#pragma unroll
+            for (int tile = 0; tile < kStepTiles; ++tile) {
+                const int key = (s_begin + i) * kKeyStep + tile * 16 + half * 8;
+                u32x4_t *v = reinterpret_cast<u32x4_t *>(vl + lds_value_offset(tile >> 1, tile & 1, half, dim));
+                if (key + 8 > n) *v &= value_keep(key, n);
+            }
+            __syncthreads();
+        }
         step_body(i + 1 < steps, i + 2 == steps && last_part, (i & 1) != 0, i, xa, xb, tail_lane);
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct)
@@ -1011,6 +1035,11 @@ __global__ __launch_bounds__(KG * 64, 2) void prefill_wave_attention_kernel(Pref
                 const bool keep = key <= my_token && key < n;
 #pragma unroll
                 for (int ct = 0; ct < CT; ++ct) x[ct][e] = keep ? x[ct][e] : -INFINITY;
+            }
+            if (t0 + kQueryBlock > n) {  // uniform: the last cache block is partly filled
+                const u32x4_t keep = value_keep(s * kWaveStep + kg * 8, n);
+#pragma unroll
+                for (int c = 0; c < 8; ++c) vf[c] = __builtin_bit_cast(half8_t, __builtin_bit_cast(u32x4_t, vf[c]) & keep);
             }
         }
         // Lazy rescale, as in prefill_attention_kernel: the reference moves
