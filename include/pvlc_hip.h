@@ -377,12 +377,13 @@ typedef struct pvlc_hip_paged_decode_args {
  * streaming launch (partitions longer than 384 tokens, or ragged cache_lens
  * with more than 512 workgroups of one (partition, kv head, sequence)) may
  * lengthen it on the device, to at most twice this and at most 4096 tokens, so
- * the items spread evenly over the compute units; it records the partition it
- * used in the workspace word after the error word
+ * the items spread evenly over the compute units
  * (pvlc_hip_paged_decode_streaming_partition gives the same choice on the
  * host).  Other launches, and ragged batches of more than 2048 sequences (more
  * than the streaming kernel numbers), run one workgroup per (partition, kv
- * head, sequence) at this partition, with the in-kernel merge. */
+ * head, sequence) at this partition, with the in-kernel merge.  Every ragged
+ * and every streaming automatic launch records the partition it used in the
+ * workspace word after the error word. */
 uint32_t pvlc_hip_paged_decode_partition(uint32_t num_seqs, uint32_t max_context);
 /* The partition an automatic streaming launch over these ragged cache lengths
  * (rows cached before the append; host memory, num_seqs entries) settles on, on

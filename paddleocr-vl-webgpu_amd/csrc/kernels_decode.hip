@@ -65,7 +65,7 @@ struct DecodeParams {
     float *part_ml;     // [seq][kv head][part_stride][8 heads][2]: max (log2 units), sum
     uint32_t *counters; // [seq][kv head]
     uint32_t *error_word;
-    uint32_t *partition_word;  // streaming, automatic partition: the one used (else null)
+    uint32_t *partition_word;  // streaming or ragged, automatic partition: receives the one used (else null)
     uint32_t compute_units;    // streaming: compute units of the device
     float scale_log2;   // log2(e)/sqrt(128)
     // f32 operands (pvlc_hip_paged_decode_f32io): query, new key and value,
@@ -758,8 +758,8 @@ __device__ inline uint32_t wave_inclusive_scan(uint32_t x) {
 template <int WAVES, int PAIRS, bool F32IO, bool KEYS_FIRST>
 __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_kernel(
     uint16_t *key_cache, uint16_t *value_cache, const int32_t *cache_lens, const int32_t *block_tables,
-    uint32_t uniform_cache_len, uint32_t max_blocks_per_seq, uint32_t num_blocks, uint32_t partition_tokens,
-    uint32_t max_parts, DecodeParams p) {
+    uint32_t uniform_cache_len, uint32_t max_blocks_per_seq, uint32_t num_blocks, uint32_t partition_and_parts,
+    uint32_t *partition_word, DecodeParams p) {
     p.key_cache = key_cache;
     p.value_cache = value_cache;
     p.cache_lens = cache_lens;
@@ -767,11 +767,19 @@ __global__ __launch_bounds__(WAVES * 64, 2) void paged_decode_kernel(
     p.uniform_cache_len = uniform_cache_len;
     p.max_blocks_per_seq = max_blocks_per_seq;
     p.num_blocks = num_blocks;
-    p.partition_tokens = partition_tokens;
-    p.max_parts = max_parts;
+    p.partition_tokens = partition_and_parts & 0xffffu;  // (at most 4096 tokens, 64 parts)
+    p.max_parts = partition_and_parts >> 16;
     const uint32_t part = blockIdx.x;
     const uint32_t g = blockIdx.y;  // kv head
     const uint32_t s = blockIdx.z;  // sequence (or layer)
+    // A ragged automatic launch leaves the partition it ran with where the
+    // streaming kernel leaves its own (uniform lengths: null).  Written before
+    // the loads, through a preloaded pointer: at the end of the first or the
+    // last workgroup it cost 13 sequences up to 2010 rows 0.1-0.2 us of 8.5.
+    if ((part | g | s) == 0 && partition_word != nullptr && threadIdx.x == 0) {
+        partition_word[0] = p.partition_tokens;
+        partition_word[1] = kTargetWorkgroups;  // the compute units the plan assumes
+    }
     const int64_t len = checked_cache_len(
         p, p.cache_lens ? load_const(p.cache_lens, s) : static_cast<int64_t>(p.uniform_cache_len));
     if (len < 0) {
@@ -1146,11 +1154,13 @@ int launch_paged_decode_kernels(const DecodeLaunch &launch, DecodeParams &p, hip
         if (p.rotate_query)                                                                                     \
             hipLaunchKernelGGL((paged_decode_kernel<W, PR, F32IO, false>), grid, dim3((W) * 64), 0, st,         \
                                p.key_cache, p.value_cache, p.cache_lens, p.block_tables, p.uniform_cache_len,   \
-                               p.max_blocks_per_seq, p.num_blocks, p.partition_tokens, p.max_parts, p);         \
+                               p.max_blocks_per_seq, p.num_blocks, p.partition_tokens | p.max_parts << 16,      \
+                               p.partition_word, p);                                                            \
         else                                                                                                    \
             hipLaunchKernelGGL((paged_decode_kernel<W, PR, F32IO, true>), grid, dim3((W) * 64), 0, st,          \
                                p.key_cache, p.value_cache, p.cache_lens, p.block_tables, p.uniform_cache_len,   \
-                               p.max_blocks_per_seq, p.num_blocks, p.partition_tokens, p.max_parts, p);         \
+                               p.max_blocks_per_seq, p.num_blocks, p.partition_tokens | p.max_parts << 16,      \
+                               p.partition_word, p);                                                            \
     } while (0)
     switch (launch.waves) {
         case 1: PVLC_DECODE_LAUNCH(1, 1); break;

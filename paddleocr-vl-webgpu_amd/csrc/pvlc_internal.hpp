@@ -155,7 +155,8 @@ struct DecodeLaunch {
     // Streaming regime with an automatic partition: the persistent kernel may
     // lengthen the partition to fill its last round of items and writes the
     // partition it used here for the merge kernel, and the compute units it
-    // assumed in the next word (null: partition_tokens as is).
+    // assumed in the next word (null: partition_tokens as is).  A ragged
+    // automatic launch of the single-shot kernel records its partition here too.
     uint32_t *partition_word;
     // f32 operands instead of args' fp16 query, new key and value, output
     // (null: the fp16 ones).

@@ -307,9 +307,10 @@ pvlc_hip_status launch_decode_state(const pvlc_hip_paged_decode_args *a, uint32_
                         state.error_word,
                         nullptr,
                         f32};
-    // An automatic streaming launch records the partition it settled on and
-    // the compute units it assumed in the two status words.
-    if (streaming && a->partition_tokens == 0) launch.partition_word = state.status_words;
+    // An automatic launch that streams or has ragged lengths records the
+    // partition it settled on and the compute units it assumed in the two
+    // status words.
+    if ((streaming || a->cache_lens) && a->partition_tokens == 0) launch.partition_word = state.status_words;
     const int e = launch_paged_decode(launch, stream);
     if (e != 0) return hip_fail(static_cast<hipError_t>(e), "paged decode launch");
     if (launches_out) *launches_out = streaming ? 2u : 1u;  // persistent kernel + merge kernel, or one kernel

@@ -124,3 +124,22 @@ def test_both_regimes_share_a_workspace():
     for rep, partition in enumerate([16, 256, 0, 16, 64, 256]):
         log(f"case: shared workspace, partition {partition}")
         batch.check(False, ws, f"partition {partition}, call {rep}", partition)
+
+
+def test_automatic_launches_record_their_partition():
+    """Ragged automatic launches of either regime over one workspace leave the partition they ran with in the word after
+    the error word (so never an earlier launch's), the first sequence refused or not; an explicit partition leaves it."""
+    words = lambda: ws[4:12].cpu().numpy().view(np.uint32)  # noqa: E731
+    ws = workspace(64, 1300)  # the largest of the launches below
+    for lens, max_context, streams in [([2, 0, 13], 16, False), ([1299] * 64, 1300, True), ([1999, 5, 300], 2010, False),
+                                       ([-5, 700], 701, False), ([1299] * 64, 1300, True), ([40] * 5, 300, False)]:
+        log(f"case: recorded partition {len(lens)} seqs max_context={max_context}")
+        assert pvlc.decode_workspace_bytes(len(lens), max_context) <= ws.numel()
+        pvlc.workspace_init(ws, 256)  # the error word of the refused sequence
+        batch = Batch(lens, max_context, len(lens))
+        batch.check(False, ws, f"{len(lens)} seqs")
+        plan, (chosen, units) = pvlc.decode_partition(len(lens), max_context), (int(w) for w in words())
+        assert units > 0 and chosen == pvlc.decode_streaming_partition(np.array(lens, np.int32), max_context, units)
+        assert streams or chosen == plan
+        batch.check(False, ws, "explicit", 32 if max_context < 500 else 512)
+        assert int(words()[0]) == chosen
