@@ -398,7 +398,10 @@ uint32_t pvlc_hip_paged_decode_partition(uint32_t num_seqs, uint32_t max_context
  * 32-key chunks, runtime-core lib.rs:2889-2978.) */
 uint32_t pvlc_hip_paged_decode_streaming_partition(const int32_t *cache_lens, uint32_t num_seqs, uint32_t max_context,
                                                    uint32_t compute_units);
-/* Workspace for split-K partials, merge counters and the device error word. */
+/* Workspace for split-K partials, merge counters and the device error word.
+ * Zeroed once, it serves stream-ordered launches of any shapes whose sizes it
+ * holds, in any order, up to 2048 sequences each; launches of more sequences
+ * keep a workspace for their own number. */
 size_t pvlc_hip_paged_decode_workspace_bytes(uint32_t num_seqs, uint32_t max_context, uint32_t partition_tokens);
 /* Zero a workspace on `stream` (a fill kernel; safe under graph capture). */
 pvlc_hip_status pvlc_hip_workspace_init(void *workspace, size_t workspace_bytes, void *stream);

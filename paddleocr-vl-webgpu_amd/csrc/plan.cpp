@@ -405,7 +405,11 @@ DecodeWorkspace decode_workspace_layout(uint32_t num_seqs, uint32_t max_parts) {
     const size_t units = static_cast<size_t>(num_seqs) * kKvHeads * w.part_stride;
     w.error_offset = 0;
     w.counters_offset = 256;
-    w.part_ml_offset = align(w.counters_offset + static_cast<size_t>(num_seqs) * kKvHeads * sizeof(uint32_t));
+    // Room for the counters of kMaxRaggedSeqs sequences whatever the launch
+    // has: the partials of a smaller launch that shares the workspace would
+    // otherwise lie on a larger one's counters, which are never cleared.
+    const size_t counted = num_seqs > kMaxRaggedSeqs ? num_seqs : kMaxRaggedSeqs;
+    w.part_ml_offset = align(w.counters_offset + counted * kKvHeads * sizeof(uint32_t));
     w.part_o_offset = align(w.part_ml_offset + units * 2 * kGroup * sizeof(float));
     w.total = align(w.part_o_offset + units * kGroup * kHeadDim * sizeof(float));
     return w;

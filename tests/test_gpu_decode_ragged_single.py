@@ -143,3 +143,18 @@ def test_automatic_launches_record_their_partition():
         assert streams or chosen == plan
         batch.check(False, ws, "explicit", 32 if max_context < 500 else 512)
         assert int(words()[0]) == chosen
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_batches_of_changing_size_share_a_workspace(f32):
+    """A serving loop keeps one workspace, zeroed once, while its batch grows and shrinks: the partials of a small batch
+    must not lie where a larger one counts arrivals.  Single launches of 3 to 256 sequences, streaming ones between."""
+    batches = [Batch([2000 - 37 * i for i in range(3)], 2010, 31), Batch([383 - 5 * i for i in range(40)], 400, 32),
+               Batch([900 - 11 * i for i in range(64)], 1000, 33), Batch([96 - i % 17 for i in range(256)], 97, 34),
+               Batch([383, 384, 5] * 42 + [20, 0], 385, 35)]
+    import torch
+    ws = torch.empty(max(pvlc.decode_workspace_bytes(len(b.lens), b.max_context) for b in batches), dtype=torch.uint8, device="cuda")
+    pvlc.workspace_init(ws, ws.numel())
+    for rep, i in enumerate([0, 1, 0, 3, 2, 4, 1, 3, 0, 4]):
+        log(f"case: one workspace, batch of {len(batches[i].lens)}, call {rep} f32={f32}")
+        batches[i].check(f32, ws, f"batch of {len(batches[i].lens)}, call {rep}")
