@@ -281,19 +281,15 @@ constexpr uint32_t prefill_pair_segments(uint32_t w, uint32_t qblocks, uint32_t 
     return n;
 }
 // Workspace of the pair schedule: an arrival counter per (pair, kv head),
-// then two partial slabs each; 0 when the blocks are short enough.  The
-// counters have room for those of a prompt of kPrefillCountedTokens, so that
-// prompts of different lengths may share a workspace: the partials of a shorter
-// one never lie on the counters of a longer one, which must be zero.
-constexpr uint32_t kPrefillCountedTokens = 65536;
+// then two partial slabs each; 0 when the blocks are short enough.
 struct PrefillWorkspace {
     size_t partial_offset, total;
 };
 inline PrefillWorkspace prefill_workspace_layout(uint32_t tokens) {
     const uint32_t qblocks = (tokens + 15u) / 16u;
     if (tokens == 0 || prefill_max_steps(qblocks) <= kPrefillSplitSteps) return {0, 0};
-    const uint32_t items = 2u * prefill_pairs(qblocks), counted = 2u * prefill_pairs(kPrefillCountedTokens / 16u);
-    const size_t counters = (static_cast<size_t>(items > counted ? items : counted) * 4 + 255) / 256 * 256;
+    const uint32_t items = 2u * prefill_pairs(qblocks);
+    const size_t counters = (static_cast<size_t>(items) * 4 + 255) / 256 * 256;
     return {counters, counters + static_cast<size_t>(items) * 2 * kPrefillPartialFloats * 4};
 }
 int launch_gemv_f16(const uint16_t *weights, const float *vector, float *out, uint32_t rows, uint32_t columns,
