@@ -477,7 +477,7 @@ typedef struct pvlc_hip_paged_prefill_args {
     void *workspace;          /* optional, 256-byte aligned, zeroed once (pvlc_hip_workspace_init): split-K schedule
                                  of long prompts (their long query blocks split over two workgroups and merged);
                                  NULL, or a shorter prompt: every query block in its own workgroups.  Launches that
-                                 share one workspace must be stream-ordered. */
+                                 share one workspace, of any prompt lengths, must be stream-ordered. */
     uint64_t workspace_bytes; /* at least pvlc_hip_paged_prefill_workspace_bytes(tokens) when workspace is given */
 } pvlc_hip_paged_prefill_args;
 

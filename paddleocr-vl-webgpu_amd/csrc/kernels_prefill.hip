@@ -77,7 +77,7 @@ struct PrefillParams {
     uint32_t *error_word;
     float scale_log2;
     // split-K pair schedule (prefill_attention_kernel)
-    uint32_t *counters;  // [pair][kv head]
+    uint32_t *counters;  // [pair][kv head], cleared by the append kernel (null: no pair schedule)
     float *partials;     // [pair][kv head][2 parts][kPrefillPartialFloats]
     // f32 operands (pvlc_hip_paged_prefill_f32io): query, key, value, output;
     // null for the fp16 entry point.
@@ -240,6 +240,14 @@ __global__ __launch_bounds__(kAppendThreads) void prefill_rope_append_kernel(Pre
         } else {
             for (uint32_t tt = 0; tt < ntok; ++tt) dst[tt] = sv[tt][hh * kHeadDim + d];
         }
+    }
+    if (p.counters && i == 0) {
+        // The pair schedule's arrival counters (one per block, and one more
+        // for an odd number) start at zero whatever lay there: a workspace may
+        // have served a shorter prompt, whose partials begin where a longer
+        // one's counters are.
+        p.counters[b] = 0;
+        if (b + 1 == gridDim.x && (gridDim.x & 1u) != 0) p.counters[b + 1] = 0;
     }
     if (p.qrot) {
         // (token, head, 8-dim chunk) items of the block's tokens
@@ -1505,13 +1513,19 @@ int launch_prefill(const pvlc_hip_paged_prefill_args *a, void *stream, const Pre
         else hipLaunchKernelGGL(prefill_short_kernel<false>, grid, threads, 0, st, p);
         return static_cast<int>(hipGetLastError());
     }
+    const bool paired = a->workspace != nullptr && a->tokens > kPrefillWaveTokens;
+    if (paired) {
+        const PrefillWorkspace ws = prefill_workspace_layout(a->tokens);
+        p.counters = static_cast<uint32_t *>(a->workspace);
+        p.partials = reinterpret_cast<float *>(static_cast<unsigned char *>(a->workspace) + ws.partial_offset);
+    }
     const dim3 append_grid((a->tokens + kBlockTokens - 1) / kBlockTokens);
     if (f32) hipLaunchKernelGGL(prefill_rope_append_kernel<true>, append_grid, dim3(kAppendThreads), 0, st, p);
     else hipLaunchKernelGGL(prefill_rope_append_kernel<false>, append_grid, dim3(kAppendThreads), 0, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return static_cast<int>(e);
     const unsigned qblocks = (a->tokens + kQueryBlock - 1) / kQueryBlock;
-    if (a->workspace == nullptr || a->tokens <= kPrefillWaveTokens) {
+    if (!paired) {
         // 1 head and 2 waves a workgroup while the prompt is short (16
         // workgroups a query block), 2 heads and 4 waves beyond.  N=211 f16:
         // 9.2 us against 10.5, 700: 14.5 against 14.8, 1157: 24.5 against
@@ -1527,9 +1541,6 @@ int launch_prefill(const pvlc_hip_paged_prefill_args *a, void *stream, const Pre
         }
         return static_cast<int>(hipGetLastError());
     }
-    const PrefillWorkspace ws = prefill_workspace_layout(a->tokens);
-    p.counters = static_cast<uint32_t *>(a->workspace);
-    p.partials = reinterpret_cast<float *>(static_cast<unsigned char *>(a->workspace) + ws.partial_offset);
     const unsigned grid = prefill_pair_workgroups(qblocks);
     if (f32) hipLaunchKernelGGL(prefill_attention_kernel<true>, dim3(grid), dim3(kWaves * 64), 0, st, p);
     else hipLaunchKernelGGL(prefill_attention_kernel<false>, dim3(grid), dim3(kWaves * 64), 0, st, p);
