@@ -18,7 +18,7 @@
 // GEMM stage of the activations is one contiguous 16 KiB run.
 // Kernel 2 (GEMM): one template from 128 x 192 down to 16 x 16 output tiles;
 // the host picks the tile by a cost that counts, per compute unit, the matrix
-// time and the bytes through its load path (choose_tile below).  The waves of
+// time and the bytes through its load path (choose_projection_tile).  The waves of
 // a workgroup own rows of the tile (activation fragments straight from the
 // planes into registers, no byte read twice) and share its weight columns,
 // which move by direct global-to-LDS loads in whole 128-byte lines; small
@@ -38,7 +38,6 @@ namespace {
 constexpr int kSplitThreads = 256;
 constexpr int kSplitRows = 8;  // rows per split workgroup: 8 x 16 bytes = one 128-byte line per chunk
 constexpr int kTileM = kProjectionTileRows, kTileK = kProjectionStepK;
-constexpr uint32_t kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 constexpr int kTileElems = kTileM * kTileK;  // fp16 elements of one 128 x 32 operand tile
 constexpr int kBlockElems = 2 * kTileElems;  // one activation block: hi and lo planes
 // s_waitcnt immediate (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4,
@@ -162,13 +161,7 @@ template <int U, int ELEMS> __device__ __forceinline__ uint16_t *weight_ring() {
 // Inside the block, generations of `gen` columns: all row tiles of the block
 // for columns [g gen, g gen + gen), row-major, so the workgroups resident at
 // once share both operands in the XCD's L2.
-constexpr uint32_t kXcdUnits = 32;      // compute units of one XCD
-constexpr uint32_t kXcdResident = 64;   // workgroups one XCD runs at once (two per compute unit)
-struct TileOrder {
-    uint32_t row_tiles, col_tiles, col_groups, gen;
-};
-
-__device__ inline bool ordered_tile(const TileOrder &o, uint32_t b, uint32_t *mt, uint32_t *nt) {
+__device__ inline bool ordered_tile(const ProjectionOrder &o, uint32_t b, uint32_t *mt, uint32_t *nt) {
     const uint32_t x = b % kXcds, idx = b / kXcds;
     const uint32_t row_groups = kXcds / o.col_groups;
     const uint32_t xr = x / o.col_groups, xc = x % o.col_groups;
@@ -229,7 +222,7 @@ template <int RB, int RW, int CB, int KG, int S, int AD, int MIN_WAVES>
 __global__ __launch_bounds__(RW *KG * 64, MIN_WAVES) void projection_gemm_kernel(
     const uint16_t *__restrict__ tiles, const int32_t *__restrict__ exponents, const uint16_t *__restrict__ weight,
     const float *__restrict__ bias, float *__restrict__ out, uint32_t rows, uint32_t k_width, uint32_t n_width,
-    TileOrder order) {
+    ProjectionOrder order) {
     typedef int int4_t __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) void *lds_ptr;
     constexpr int kTM = RB * RW * 16, kTN = CB * 16;
@@ -256,9 +249,10 @@ __global__ __launch_bounds__(RW *KG * 64, MIN_WAVES) void projection_gemm_kernel
     const uint16_t *a_base = tiles + static_cast<size_t>(m0 / kTileM) * steps * kBlockElems;
     const uint32_t a_lane = (kg * kTileM + m0 % kTileM + row16) * 8;
     // Lane l of a weight load fills LDS place l % 8 of row l / 8 (byte
-    // offsets, which choose_tile keeps within 32 bits; 8-element chunks for CB
-    // = 1, within 32 bits at any depth; w_tail for an odd last stage, whose
-    // second half re-reads the first and is not used).
+    // offsets, which choose_projection_tile keeps within 32 bits; 8-element
+    // chunks for CB = 1, within 32 bits up to a depth of 2^31, whose planes of
+    // 128 rows or more would take a terabyte; w_tail for an odd last stage,
+    // whose second half re-reads the first and is not used).
     const uint32_t chunk = (lane & 7) ^ (lane >> 3), unit = CB == 1 ? 1 : 16;
     uint32_t w_lane[2], w_tail[2];
 #pragma unroll
@@ -419,79 +413,16 @@ __global__ __launch_bounds__(RW *KG * 64, MIN_WAVES) void projection_gemm_kernel
     }
 }
 
-// The tiles, by preference on equal cost.
-struct TileShape {
-    uint32_t rows, cols;
-};
-constexpr TileShape kShapes[] = {{128, 192}, {128, 160}, {128, 128}, {128, 64}, {64, 64}, {128, 96},
-                                  {64, 96},   {32, 64},   {16, 64},   {16, 32},  {16, 16}};
-constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
-
-// Order of the tiles: the column grouping that gives the busiest compute unit
-// the fewest tiles (the XCDs finish together), then the fewest operand bytes
-// of an XCD's block (a row of activations is twice a row of weights), and
-// generations of columns sized so that one generation is what an XCD runs at
-// once.  *block receives the tiles of the largest block.  (The exact number of
-// tiles in the first place cost bytes for nothing: 1600 rows, o 29.6 us against
-// 26.7, down 37.1 against 34.7, four or eight column groups against one.)
-TileOrder tile_order(uint32_t row_tiles, uint32_t col_tiles, const TileShape &t, uint64_t *block) {
-    TileOrder best{row_tiles, col_tiles, 1, 1};
-    uint64_t best_turns = UINT64_MAX, best_bytes = UINT64_MAX;
-    for (uint32_t gc = 1; gc <= kXcds; gc *= 2) {
-        const uint32_t gr = kXcds / gc;
-        const uint64_t rb = (row_tiles + gr - 1) / gr, cb = (col_tiles + gc - 1) / gc;
-        const uint64_t turns = (rb * cb + kXcdUnits - 1) / kXcdUnits, bytes = rb * t.rows * 2 + cb * t.cols;
-        if (turns < best_turns || (turns == best_turns && bytes < best_bytes)) {
-            best_turns = turns;
-            best_bytes = bytes;
-            best.col_groups = gc;
-            *block = rb * cb;
-        }
-    }
-    const uint32_t gr = kXcds / best.col_groups, rb = (row_tiles + gr - 1) / gr;
-    best.gen = kXcdResident / rb > 0 ? kXcdResident / rb : 1;
-    return best;
-}
-
-// The tile of a launch: the least clocks of the busiest compute unit per
-// 32-deep step, (tiles it runs) x max(matrix time, load time) with rows cols /
-// 32 clocks of MFMAs (hi and lo, 4096 FLOP per clock) and 2 rows + cols clocks
-// of loads (64 bytes per clock) a tile; on ties the earlier in the list (two
-// 64 x 64 tiles a unit overlap, one 128 x 96 does not: 300 rows of gate|up 17.5
-// against 19.1 us).  The unit's tiles are those of the largest XCD block over
-// its 32 units.  Against every tile timed at 16 to 4096 rows of the decoder's
-// projections this picks the fastest or one within 3% of it.  What the 96
-// column tiles save over the others: 400 rows, gate|up 23.3 -> 20.9 us; 900
-// rows, q|k|v 23.5 -> 20.8; 1157 rows, o 26.1 -> 24.0 and down 33.0 -> 30.4.
-int choose_tile(uint32_t rows, uint32_t k_width, uint32_t n_width, TileOrder *order, uint64_t *block) {
-    int best = kShapeCount - 1;
-    uint64_t best_cost = UINT64_MAX;
-    for (int i = 0; i < kShapeCount; ++i) {
-        const TileShape t = kShapes[i];
-        // The shifted last column tile needs a whole one, and a row of
-        // weights at most 2^29 bytes (32-bit offsets over 8 rows); the 16 x 16
-        // tile takes any.
-        if (i + 1 < kShapeCount && (n_width < t.cols || k_width > 1u << 28)) continue;
-        uint64_t b = 0;
-        const TileOrder o = tile_order((rows + t.rows - 1) / t.rows, n_width / t.cols + (n_width % t.cols != 0), t, &b);
-        const uint64_t mfma = t.rows * t.cols / 32, loads = 2 * t.rows + t.cols;
-        const uint64_t cost = (b + kXcdUnits - 1) / kXcdUnits * (mfma > loads ? mfma : loads);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = i;
-            *order = o;
-            *block = b;
-        }
-    }
-    return best;
-}
-
 }  // namespace
 
 int launch_linear_projection_f16(const float *input, const uint16_t *weight, const float *bias, float *out,
                                  uint32_t rows, uint32_t k_width, uint32_t n_width, const ProjectionWorkspace &ws,
                                  void *stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
+    ProjectionOrder order{};
+    uint64_t block = 0;
+    const int shape = choose_projection_tile(rows, k_width, n_width, &order, &block);
+    if (shape < 0) return static_cast<int>(hipErrorInvalidConfiguration);  // (operands beyond any device's memory)
     const uint32_t m_tiles = (rows + kTileM - 1) / kTileM;
     const dim3 split_grid(m_tiles * (kTileM / kSplitRows));
     switch (k_width) {
@@ -502,27 +433,26 @@ int launch_linear_projection_f16(const float *input, const uint16_t *weight, con
     default: hipLaunchKernelGGL(projection_split_kernel<0>, split_grid, dim3(kSplitThreads), 0, st, input, rows, k_width, ws.tiles, ws.exponents); break;
     }
     if (hipError_t e = hipGetLastError()) return static_cast<int>(e);
-    TileOrder order;
-    uint64_t block = 0;
-    const int shape = choose_tile(rows, k_width, n_width, &order, &block);
     const dim3 grid(static_cast<uint32_t>(kXcds * block));
-#define PVLC_PROJECTION_LAUNCH(RB, RW, CB, KG, S, AD, MW)                                                          \
+#define PVLC_PROJECTION_LAUNCH(I, RB, RW, CB, KG, S, AD, MW)                                                       \
     do {                                                                                                           \
+        static_assert(kProjectionTiles[I].rows == (RB) * (RW) * 16 && kProjectionTiles[I].cols == (CB) * 16 &&     \
+                      kProjectionTiles[I].threads == (RW) * (KG) * 64, "the tile that choose_projection_tile weighed"); \
         hipLaunchKernelGGL((projection_gemm_kernel<RB, RW, CB, KG, S, AD, MW>), grid, dim3((RW) * (KG) * 64), 0, st, \
                            ws.tiles, ws.exponents, weight, bias, out, rows, k_width, n_width, order);              \
     } while (0)
-    switch (shape) {  // kShapes
-    case 0: PVLC_PROJECTION_LAUNCH(2, 4, 12, 1, 3, 3, 2); break;
-    case 1: PVLC_PROJECTION_LAUNCH(2, 4, 10, 1, 3, 3, 2); break;
-    case 2: PVLC_PROJECTION_LAUNCH(2, 4, 8, 1, 3, 3, 2); break;
-    case 3: PVLC_PROJECTION_LAUNCH(2, 4, 4, 2, 3, 3, 2); break;
-    case 4: PVLC_PROJECTION_LAUNCH(2, 2, 4, 2, 3, 3, 2); break;
-    case 5: PVLC_PROJECTION_LAUNCH(2, 4, 6, 2, 3, 3, 2); break;
-    case 6: PVLC_PROJECTION_LAUNCH(2, 2, 6, 2, 3, 3, 2); break;
-    case 7: PVLC_PROJECTION_LAUNCH(2, 1, 4, 4, 2, 4, 2); break;
-    case 8: PVLC_PROJECTION_LAUNCH(1, 1, 4, 4, 2, 4, 2); break;
-    case 9: PVLC_PROJECTION_LAUNCH(1, 1, 2, 8, 2, 4, 4); break;
-    default: PVLC_PROJECTION_LAUNCH(1, 1, 1, 8, 2, 4, 4); break;
+    switch (shape) {  // kProjectionTiles
+    case 0: PVLC_PROJECTION_LAUNCH(0, 2, 4, 12, 1, 3, 3, 2); break;
+    case 1: PVLC_PROJECTION_LAUNCH(1, 2, 4, 10, 1, 3, 3, 2); break;
+    case 2: PVLC_PROJECTION_LAUNCH(2, 2, 4, 8, 1, 3, 3, 2); break;
+    case 3: PVLC_PROJECTION_LAUNCH(3, 2, 4, 4, 2, 3, 3, 2); break;
+    case 4: PVLC_PROJECTION_LAUNCH(4, 2, 2, 4, 2, 3, 3, 2); break;
+    case 5: PVLC_PROJECTION_LAUNCH(5, 2, 4, 6, 2, 3, 3, 2); break;
+    case 6: PVLC_PROJECTION_LAUNCH(6, 2, 2, 6, 2, 3, 3, 2); break;
+    case 7: PVLC_PROJECTION_LAUNCH(7, 2, 1, 4, 4, 2, 4, 2); break;
+    case 8: PVLC_PROJECTION_LAUNCH(8, 1, 1, 4, 4, 2, 4, 2); break;
+    case 9: PVLC_PROJECTION_LAUNCH(9, 1, 1, 2, 8, 2, 4, 4); break;
+    default: PVLC_PROJECTION_LAUNCH(10, 1, 1, 1, 8, 2, 4, 4); break;
     }
 #undef PVLC_PROJECTION_LAUNCH
     return static_cast<int>(hipGetLastError());

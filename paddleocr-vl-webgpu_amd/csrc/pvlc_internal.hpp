@@ -197,6 +197,83 @@ inline ProjectionWorkspaceLayout projection_workspace_layout(uint32_t rows, uint
     const size_t tiles = padded * k_width * 4;  // two fp16 planes
     return {tiles, tiles + (padded * 4 + 255) / 256 * 256};
 }
+// The tiles of the projection GEMM (kernels_projection.hip) and the threads of
+// their workgroups, by preference on equal cost.
+struct ProjectionTile {
+    uint32_t rows, cols, threads;
+};
+constexpr ProjectionTile kProjectionTiles[] = {{128, 192, 256}, {128, 160, 256}, {128, 128, 256}, {128, 64, 512},
+                                               {64, 64, 256},   {128, 96, 512},  {64, 96, 256},   {32, 64, 256},
+                                               {16, 64, 256},   {16, 32, 512},   {16, 16, 512}};
+constexpr int kProjectionTileCount = sizeof(kProjectionTiles) / sizeof(kProjectionTiles[0]);
+constexpr uint32_t kXcds = 8;           // MI355X: 8 XCDs, each with its own L2
+constexpr uint32_t kXcdUnits = 32;      // compute units of one XCD
+constexpr uint32_t kXcdResident = 64;   // workgroups one XCD runs at once (two per compute unit)
+struct ProjectionOrder {
+    uint32_t row_tiles, col_tiles, col_groups, gen;
+};
+
+// Order of the tiles: the column grouping that gives the busiest compute unit
+// the fewest tiles (the XCDs finish together), then the fewest operand bytes
+// of an XCD's block (a row of activations is twice a row of weights), and
+// generations of columns sized so that one generation is what an XCD runs at
+// once.  *block receives the tiles of the largest block.  (The exact number of
+// tiles in the first place cost bytes for nothing: 1600 rows, o 29.6 us against
+// 26.7, down 37.1 against 34.7, four or eight column groups against one.)
+inline ProjectionOrder projection_order(uint32_t row_tiles, uint32_t col_tiles, const ProjectionTile &t, uint64_t *block) {
+    ProjectionOrder best{row_tiles, col_tiles, 1, 1};
+    uint64_t best_turns = UINT64_MAX, best_bytes = UINT64_MAX;
+    for (uint32_t gc = 1; gc <= kXcds; gc *= 2) {
+        const uint32_t gr = kXcds / gc;
+        const uint64_t rb = (row_tiles + gr - 1) / gr, cb = (col_tiles + gc - 1) / gc;
+        const uint64_t turns = (rb * cb + kXcdUnits - 1) / kXcdUnits, bytes = rb * t.rows * 2 + cb * t.cols;
+        if (turns < best_turns || (turns == best_turns && bytes < best_bytes)) {
+            best_turns = turns;
+            best_bytes = bytes;
+            best.col_groups = gc;
+            *block = rb * cb;
+        }
+    }
+    const uint32_t gr = kXcds / best.col_groups, rb = (row_tiles + gr - 1) / gr;
+    best.gen = kXcdResident / rb > 0 ? kXcdResident / rb : 1;
+    return best;
+}
+
+// The tile of a launch: the least clocks of the busiest compute unit per
+// 32-deep step, (tiles it runs) x max(matrix time, load time) with rows cols /
+// 32 clocks of MFMAs (hi and lo, 4096 FLOP per clock) and 2 rows + cols clocks
+// of loads (64 bytes per clock) a tile; on ties the earlier in the list (two
+// 64 x 64 tiles a unit overlap, one 128 x 96 does not: 300 rows of gate|up 17.5
+// against 19.1 us).  The unit's tiles are those of the largest XCD block over
+// its 32 units.  Against every tile timed at 16 to 4096 rows of the decoder's
+// projections this picks the fastest or one within 3% of it.  What the 96
+// column tiles save over the others: 400 rows, gate|up 23.3 -> 20.9 us; 900
+// rows, q|k|v 23.5 -> 20.8; 1157 rows, o 26.1 -> 24.0 and down 33.0 -> 30.4.
+// The grid, 8 times the largest block, keeps under 2^32 threads, which few rows
+// of 2^30 or more columns exceed with the small tiles.  -1: no tile does.
+inline int choose_projection_tile(uint32_t rows, uint32_t k_width, uint32_t n_width, ProjectionOrder *order, uint64_t *block) {
+    int best = -1;
+    uint64_t best_cost = UINT64_MAX;
+    for (int i = 0; i < kProjectionTileCount; ++i) {
+        const ProjectionTile t = kProjectionTiles[i];
+        // The shifted last column tile needs a whole one, and a row of
+        // weights at most 2^29 bytes (32-bit offsets over 8 rows); the 16 x 16
+        // tile takes any.
+        if (i + 1 < kProjectionTileCount && (n_width < t.cols || k_width > 1u << 28)) continue;
+        uint64_t b = 0;
+        const ProjectionOrder o = projection_order(rows / t.rows + (rows % t.rows != 0), n_width / t.cols + (n_width % t.cols != 0), t, &b);
+        const uint64_t mfma = t.rows * t.cols / 32, loads = 2 * t.rows + t.cols;
+        const uint64_t cost = (b + kXcdUnits - 1) / kXcdUnits * (mfma > loads ? mfma : loads);
+        if (cost < best_cost && b * kXcds * t.threads < 1ull << 32) {
+            best_cost = cost;
+            best = i;
+            *order = o;
+            *block = b;
+        }
+    }
+    return best;
+}
+
 int launch_linear_projection_f16(const float *input, const uint16_t *weight, const float *bias, float *out,
                                  uint32_t rows, uint32_t k_width, uint32_t n_width, const ProjectionWorkspace &ws,
                                  void *stream);

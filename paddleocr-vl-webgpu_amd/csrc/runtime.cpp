@@ -838,8 +838,8 @@ pvlc_hip_status pvlc_hip_linear_projection_f16(const float *input, const uint16_
                        "projection geometry must be positive with widths a multiple of 4");
     if (input_width % 32 != 0)
         return invalid(PVLC_HIP_INV_INVALID_DECODER_GEOMETRY, "device projection needs input_width a multiple of 32");
-    // Outputs of more than 2^24 tiles of 128 x 128 exceed any device's memory; below, every tile the launch may
-    // choose keeps the grid under 2^32 threads.
+    // Outputs of more than 2^24 tiles of 128 x 128 exceed any device's memory; below, choose_projection_tile keeps
+    // the grid under 2^32 threads.
     const uint64_t out_tiles = (static_cast<uint64_t>(rows) + 127) / 128 * ((static_cast<uint64_t>(output_width) + 127) / 128);
     if (rows > 65535u * 128u || out_tiles >= (1u << 24))
         return invalid(PVLC_HIP_INV_INVALID_DECODER_GEOMETRY, "projection rows or output tiles exceed the grid");
