@@ -333,6 +333,9 @@ __global__ __launch_bounds__(RW *KG * 64, MIN_WAVES) void projection_gemm_kernel
             b[cb] = *reinterpret_cast<const half8_t *>(sw + (r * 8 + (c ^ (r & 7))) * 8);
         }
         load_w(st + S - 1, weight_ring<kNext, kSlotElems>(), H % 2 ? kW0 : 0, H % 2 ? kWLoads : kW0);
+        // Where the wait for a stage's weights allows no more than the activation
+        // loads behind them (S = 2), the two keep this order.
+        if constexpr (H % 2 == 1 && kWaitStage > (2 * S - 4) * kHalfLoads) __builtin_amdgcn_sched_barrier(0);
         load_a(2 * st + H % 2 + AD - 1, f[(H + AD - 1) % AD]);
         __builtin_amdgcn_sched_barrier(0);
         if (2 * st + H % 2 < steps) {  // uniform
