@@ -507,7 +507,9 @@ pvlc_hip_status pvlc_hip_paged_prefill_f32io(const pvlc_hip_paged_prefill_args *
                                              const float *key, const float *value, float *out, void *stream);
 
 /* Compact [tokens][2][128] fp16 rows <-> blocked planes (bit-exact), rows
- * 0..tokens-1 of one sequence through its block table (NULL = blocks 0..). */
+ * 0..tokens-1 of one sequence through its block table (NULL = blocks 0..).
+ * Rows and planes need the alignment of their elements only (16-byte aligned
+ * ones move fastest; decode and prefill require that of planes). */
 pvlc_hip_status pvlc_hip_kv_pack_f16(const uint16_t *key_rows, const uint16_t *value_rows, uint32_t tokens,
                                      const int32_t *block_table, uint32_t num_blocks, uint16_t *key_cache,
                                      uint16_t *value_cache, void *stream);

@@ -12,6 +12,10 @@ namespace pvlc {
 namespace {
 
 typedef uint16_t u16x8_t __attribute__((ext_vector_type(8)));
+// The same in global memory: rows and planes need only their elements'
+// alignment, so the 16-byte accesses must not assume more (the instructions are
+// those of aligned ones: the target allows unaligned global accesses).
+typedef u16x8_t u16x8_any __attribute__((aligned(2)));
 
 // Both kernels: one workgroup per 16-token cache block, both heads, with the
 // block transposed through LDS, so that the rows (32 lanes on the 512 bytes of
@@ -51,8 +55,8 @@ __global__ __launch_bounds__(kMoveThreads) void kv_pack_kernel(
     for (int r = 0; r < 2; ++r) {
         const int k = i + r * kMoveThreads;  // row piece; tokens past the end repeat the last one
         const size_t src = static_cast<size_t>(t0 + min(static_cast<uint32_t>(k >> 5), ntok - 1)) * kRowElems + (k & 31) * 8;
-        kr[r] = *reinterpret_cast<const u16x8_t *>(key_rows + src);
-        vr[r] = *reinterpret_cast<const u16x8_t *>(value_rows + src);
+        kr[r] = *reinterpret_cast<const u16x8_any *>(key_rows + src);
+        vr[r] = *reinterpret_cast<const u16x8_any *>(value_rows + src);
     }
     if (!ok) {  // uniform
         if (i == 0 && error_word) atomicOr(error_word, 2u);
@@ -70,7 +74,7 @@ __global__ __launch_bounds__(kMoveThreads) void kv_pack_kernel(
     for (int r = 0; r < 2; ++r) {
         const int k = i + r * kMoveThreads;  // slab piece; the other tokens of a partial block stay as they are
         if (static_cast<uint32_t>(key_slot(k & 15)) < ntok)  // (the slot map is its own inverse)
-            *reinterpret_cast<u16x8_t *>(key_cache + block + static_cast<size_t>(k) * 8) = sk[k];
+            *reinterpret_cast<u16x8_any *>(key_cache + block + static_cast<size_t>(k) * 8) = sk[k];
     }
     // value slab row i = (head, dim): 16 tokens
     uint16_t *dst = value_cache + block + static_cast<size_t>(i) * kBlockTokens;
@@ -81,8 +85,8 @@ __global__ __launch_bounds__(kMoveThreads) void kv_pack_kernel(
             lo[t] = sv[t][i];
             hi[t] = sv[t + 8][i];
         }
-        *reinterpret_cast<u16x8_t *>(dst) = lo;
-        *reinterpret_cast<u16x8_t *>(dst + 8) = hi;
+        *reinterpret_cast<u16x8_any *>(dst) = lo;
+        *reinterpret_cast<u16x8_any *>(dst + 8) = hi;
     } else {
         for (uint32_t t = 0; t < ntok; ++t) dst[t] = sv[t][i];
     }
@@ -113,8 +117,8 @@ __global__ __launch_bounds__(kMoveThreads) void kv_unpack_kernel(
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             const size_t k = i + r * kMoveThreads;
-            kr[r] = *reinterpret_cast<const u16x8_t *>(key_cache + block + k * 8);
-            vr[r] = __builtin_bit_cast(u32x4_t, *reinterpret_cast<const u16x8_t *>(value_cache + block + k * 8));
+            kr[r] = *reinterpret_cast<const u16x8_any *>(key_cache + block + k * 8);
+            vr[r] = __builtin_bit_cast(u32x4_t, static_cast<u16x8_t>(*reinterpret_cast<const u16x8_any *>(value_cache + block + k * 8)));
         }
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
@@ -134,7 +138,7 @@ __global__ __launch_bounds__(kMoveThreads) void kv_unpack_kernel(
         if (static_cast<uint32_t>(t) >= ntok) continue;
         u16x8_t kv{};
         if (ok) kv = sk[key_piece(t, (k >> 4) & 1, k & 15)];
-        *reinterpret_cast<u16x8_t *>(key_rows + static_cast<size_t>(t0 + t) * kRowElems + (k & 31) * 8) = kv;
+        *reinterpret_cast<u16x8_any *>(key_rows + static_cast<size_t>(t0 + t) * kRowElems + (k & 31) * 8) = kv;
     }
     // Value row pieces, two tokens a thread: pair i / 32, 16 bytes i % 32.
     const int p = i >> 5, c = i & 31;
@@ -148,8 +152,8 @@ __global__ __launch_bounds__(kMoveThreads) void kv_unpack_kernel(
         }
     }
     uint16_t *dst = value_rows + static_cast<size_t>(t0 + 2 * p) * kRowElems + c * 8;
-    if (static_cast<uint32_t>(2 * p) < ntok) *reinterpret_cast<u16x8_t *>(dst) = even;
-    if (static_cast<uint32_t>(2 * p + 1) < ntok) *reinterpret_cast<u16x8_t *>(dst + kRowElems) = odd;
+    if (static_cast<uint32_t>(2 * p) < ntok) *reinterpret_cast<u16x8_any *>(dst) = even;
+    if (static_cast<uint32_t>(2 * p + 1) < ntok) *reinterpret_cast<u16x8_any *>(dst + kRowElems) = odd;
 }
 
 }  // namespace

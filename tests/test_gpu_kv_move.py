@@ -48,3 +48,30 @@ def test_pack_and_unpack_move_every_bit(tokens, table):
         got = from_dev(back)
         np.testing.assert_array_equal(got[:tokens * W], rows)
         assert np.all(got[tokens * W:] == 7), "unpack wrote past the rows"
+
+
+@pytest.mark.parametrize("tokens", [16, 31, 300])
+@pytest.mark.parametrize("shift", [1, 4])
+def test_operands_need_their_elements_alignment_only(tokens, shift):
+    """Rows and planes that begin 2 or 8 bytes after a 16-byte boundary."""
+    import torch
+    log(f"case: kv move tokens={tokens} shifted by {2 * shift} bytes")
+    rng = np.random.default_rng(tokens)
+    used = (tokens + 15) // 16
+    k, v = (rng.integers(0, 1 << 16, tokens * W, dtype=np.uint16) for _ in range(2))
+    planes = [rng.integers(0, 1 << 16, used * 16 * W, dtype=np.uint16) for _ in range(2)]
+    shifted = lambda a: to_dev(np.concatenate([np.zeros(shift, np.uint16), a, np.full(64, 7, np.uint16)]))[shift:]  # noqa: E731
+    d_rows, d_planes = [shifted(k), shifted(v)], [shifted(p) for p in planes]
+    backs = [shifted(np.zeros(tokens * W, np.uint16)) for _ in range(2)]
+    assert all(x.data_ptr() % 16 == 2 * shift for x in d_rows + d_planes + backs)
+    pvlc.kv_pack_f16(*d_rows, tokens, *d_planes, used)
+    pvlc.kv_unpack_f16(*d_planes, tokens, *backs, used)
+    torch.cuda.synchronize()
+    for b in range(used):
+        n = min(16, tokens - b * 16)
+        part = slice(b * 16 * W, (b * 16 + n) * W)
+        scatter_rows(*planes, k[part], v[part], n, [b])
+    for d, want in zip(d_planes + backs, planes + [k, v]):
+        got = from_dev(d)
+        np.testing.assert_array_equal(got[:-64], want)
+        assert np.all(got[-64:] == 7), "wrote past the end"
