@@ -182,8 +182,11 @@ typedef struct pvlc_hip_kv_session pvlc_hip_kv_session;
  * and a session step that fails so leaves the session terminally poisoned
  * (decoder_kv_session.rs:729-735, :513-528).  A session whose GPU work never
  * completes keeps its device buffers allocated when it is destroyed, rather
- * than freeing memory a kernel may still access.  A runtime keeps the buffers
- * of one released session (at most 64 MiB on the device and 64 MiB pinned) for
+ * than freeing memory a kernel may still access.  A live session holds its fp16
+ * cache on the device, as many bytes of pinned host memory (uploads and finish
+ * pass through it) and twice as many of ordinary memory (the rows as given, in
+ * f32).  A runtime keeps the buffers of one released session, the largest of at
+ * most 64 MiB on the device and 64 MiB pinned (so at most 128 MiB of rows), for
  * the next session they fit, until it is destroyed. */
 typedef struct pvlc_hip_runtime_options {
     int32_t device;               /* HIP device ordinal */

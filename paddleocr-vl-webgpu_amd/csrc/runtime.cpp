@@ -21,6 +21,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "pvlc_internal.hpp"
@@ -55,10 +56,10 @@ struct pvlc_hip_runtime {
     uint32_t live_sessions = 0;
     bool destroy_requested = false;
     // Buffers of a finished session, taken by the next one that they fit:
-    // allocating and freeing them took ~0.4 ms a session.  One set, of at most
-    // kMaxSpareBytes on the device and pinned each, freed with the runtime or
-    // when a session finds it too small;
-    // used under the execution lock.
+    // allocating and freeing them took ~0.4 ms a session.  One set, the larger
+    // of those given back, of at most kMaxSpareBytes on the device and pinned
+    // each (so of at most twice that in f32 rows), freed with the runtime or
+    // when a session finds it too small; used under the execution lock.
     SessionBuffers spare;
 };
 
@@ -155,7 +156,7 @@ void free_buffers(SessionBuffers &b) {
 
 // Gives the session's buffers back once the GPU work queued on the runtime
 // has completed (a bounded wait): to the runtime's spare set, or to the system
-// when that is taken, they are large, or the queue has failed.  A session
+// when that holds a larger one, they are large, or the queue has failed.  A session
 // whose work does not complete within the bound keeps its buffers allocated
 // (leaked) rather than freeing memory a kernel or a copy may still access.
 void release_buffers(pvlc_hip_kv_session *s) {
@@ -164,12 +165,10 @@ void release_buffers(pvlc_hip_kv_session *s) {
     const hipError_t e = wait_bounded(rt, false);
     if (e == hipErrorNotReady) return;
     SessionBuffers &b = s->buffers;
-    if (e == hipSuccess && rt->spare.device == nullptr && b.device != nullptr && b.pinned != nullptr &&
-        b.device_bytes <= kMaxSpareBytes && b.pinned_bytes <= kMaxSpareBytes)
-        rt->spare = std::move(b);
-    else
-        free_buffers(b);
-    b = SessionBuffers{};
+    if (e == hipSuccess && b.pinned != nullptr && b.device_bytes <= kMaxSpareBytes && b.pinned_bytes <= kMaxSpareBytes &&
+        b.device_bytes > rt->spare.device_bytes)  // (both parts grow with the capacity)
+        std::swap(b, rt->spare);
+    free_buffers(b);
 }
 
 void destroy_runtime_now(pvlc_hip_runtime *rt) {

@@ -58,3 +58,30 @@ def test_sessions_over_reused_buffers():
         else:
             del third  # dropped without finishing
     runtime.close()
+
+
+def test_the_larger_set_is_kept():
+    """Two sessions that lived side by side end in either order: the larger one's buffers serve the next large session
+    (no device memory is allocated for it), and the runtime gives everything back."""
+    import torch
+    used = lambda: base - torch.cuda.mem_get_info()[0]  # noqa: E731
+    torch.cuda.synchronize()
+    small, large, large_bytes = (5, 40), (9, 32768), 2 * 32768 * 512
+    for order in ("small first", "large first"):
+        log(f"case: session buffers kept, {order}")
+        base = torch.cuda.mem_get_info()[0]
+        runtime = pvlc.NativeRuntime(0)
+        a, b = Live(runtime, *large, seed=1), Live(runtime, *small, seed=2)
+        both = used()
+        assert both >= large_bytes
+        for x in (b, a) if order == "small first" else (a, b):
+            x.step()
+            x.finish()
+        assert large_bytes <= used() <= both
+        kept = used()
+        c = Live(runtime, *large, seed=3)
+        assert used() == kept, "a large session allocated beside the kept buffers"
+        c.step()
+        c.finish()
+        runtime.close()
+        assert used() < large_bytes
