@@ -484,7 +484,9 @@ typedef struct pvlc_hip_paged_prefill_args {
     uint64_t workspace_bytes; /* at least pvlc_hip_paged_prefill_workspace_bytes(tokens) when workspace is given */
 } pvlc_hip_paged_prefill_args;
 
-/* Bytes of the split-K prefill workspace for N tokens (0: nothing splits). */
+/* Bytes of the split-K prefill workspace for N tokens: 0 up to 2048.  It is
+ * used from 3073 tokens on; a call of 2049 to 3072 runs the same with a
+ * workspace of that size or with none (NULL), so none need be allocated. */
 size_t pvlc_hip_paged_prefill_workspace_bytes(uint32_t tokens);
 
 /* Causal prefill: rotary on Q and K, write all N K/V rows into the blocked

@@ -53,11 +53,8 @@ constexpr int kKeyStep = 64;     // keys per softmax step (4 cache blocks)
 constexpr int kStepTiles = kKeyStep / 16;
 constexpr int kWaves = 4;        // each wave: 2 of the 8 heads of the group
 constexpr float kLazyRescaleLog2 = 8.0f;  // softmax reference moves only past 2^8
-// Longest prompt of prefill_wave_attention_kernel when the caller gave a
-// workspace for the pair schedule (us, wave / pair: N=3000 f16 63.7 / 66.9,
-// f32 77.6 / 83.0; 3500 80.2 / 75.0, 97.6 / 94.7; 4096 100.5 / 86.0, 124 /
-// 112), and of its one-head form.
-constexpr uint32_t kPrefillWaveTokens = 3072, kPrefillOneHeadTokens = 768;
+// Longest prompt of the one-head form of prefill_wave_attention_kernel.
+constexpr uint32_t kPrefillOneHeadTokens = 768;
 
 struct PrefillParams {
     uint32_t tokens;

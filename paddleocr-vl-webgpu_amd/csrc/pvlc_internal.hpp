@@ -290,8 +290,8 @@ int launch_linear_projection_f16(const float *input, const uint16_t *weight, con
 // first lets the second workgroup find it complete and merge it without
 // storing its own part: config 4 at N=4096, 99.8-100.8 -> 96.6-97.3 us mean
 // per call.  The workspace is asked for when the longest block is longer than
-// kPrefillSplitSteps and used by the prompts that launch_prefill gives to this
-// schedule.  A pair whose light workgroup
+// kPrefillSplitSteps and used by prompts beyond kPrefillWaveTokens.  A pair
+// whose light workgroup
 // would take fewer than kPrefillSplitMin heavy steps at an even split is not
 // split (the light block and the heavy block run whole on the two
 // workgroups): a second segment costs its workgroup a query load, a pipeline
@@ -313,6 +313,13 @@ constexpr uint32_t kPrefillPartialFloats = 4 * 64 * 74;  // 4 waves x 64 lanes x
 constexpr uint32_t prefill_block_steps(uint32_t qb) { return qb / 4 + 1; }
 constexpr uint32_t prefill_max_steps(uint32_t qblocks) { return (qblocks - 1) / 4 + 1; }
 constexpr uint32_t prefill_pairs(uint32_t qblocks) { return (qblocks + 1) / 2; }
+// Longest prompt of prefill_wave_attention_kernel when the caller gave a
+// workspace for the pair schedule (us, wave / pair: N=3000 f16 63.7 / 66.9,
+// f32 77.6 / 83.0; 3500 80.2 / 75.0, 97.6 / 94.7; 4096 100.5 / 86.0, 124 /
+// 112).  Shorter prompts still have a workspace size (from kPrefillSplitSteps
+// on): callers compute, check and pass it, but nothing of it is touched.
+constexpr uint32_t kPrefillWaveTokens = 3072;
+static_assert(prefill_max_steps(kPrefillWaveTokens / 16 + 1) > kPrefillSplitSteps, "every paired prompt has a workspace");
 constexpr uint32_t prefill_pair_workgroups(uint32_t qblocks) { return 4u * prefill_pairs(qblocks); }
 
 struct PrefillSegment {
