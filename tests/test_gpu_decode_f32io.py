@@ -5,7 +5,8 @@ web decoder_stack_session.rs:4698-4729).
 
 - With inputs that fp16 holds exactly, the caches the f32 entry point leaves are bit-identical to the fp16 entry
   point's -- in the single-shot regime (18 layers, T=2048, the in-kernel merge), with one partition (no merge),
-  and in the streaming regime (ragged paged batch: persistent kernel + merge kernel).  Its f32 output carries
+  for a small ragged paged batch (the same regime) and in the streaming regime (a larger one: persistent kernel
+  + merge kernel).  Its f32 output carries
   the softmax weights as hi + lo fp16 pairs, so on every sequence it meets the reference's native decode policy
   against decode_gqa_f32 (max-abs 4e-4, mean 6e-5, p99 2.5e-4, relative L2 1.5e-4, cosine 0.99999;
   decoder_cached_gqa_native_contract.rs:147-158); the fp16 entry point (fp16 weights, fp16 output) stays within
@@ -96,8 +97,10 @@ def launch(case, q, nk, nv, f32, rotate_query, partition=0, uniform=False):
 @pytest.mark.parametrize("label,lens,paged,uniform,rotate_query", [
     ("18 layers T=2048 (single shot, in-kernel merge)", [2048] * 18, False, True, True),
     ("4 sequences T=40 (one partition, no merge)", [40] * 4, False, True, False),
-    ("12 ragged paged sequences (streaming + merge kernel)", [1, 17, 300, 900, 1500, 2047, 2048, 2500, 3000, 64,
-                                                               129, 777], True, False, True),
+    ("12 ragged paged sequences (one launch)", [1, 17, 300, 900, 1500, 2047, 2048, 2500, 3000, 64, 129, 777],
+     True, False, True),
+    ("36 ragged paged sequences (streaming + merge kernel)", [1, 17, 300, 900, 1500, 2047, 2048, 2500, 3000, 64,
+                                                              129, 777] * 3, True, False, True),
 ])
 def test_f32_operands_leave_the_fp16_caches_and_meet_the_native_policy(label, lens, paged, uniform, rotate_query):
     log(f"case: f32 operands vs fp16 entry point and the oracle, {label}")

@@ -110,10 +110,11 @@ def sampled_rows_match_decode(out, qr, kr, vr, n, rows, label):
         check_close(out[i], want, f"{label} row {i}")
 
 
-@pytest.mark.parametrize("n", [2049, 2100, 3000, 4096])
+@pytest.mark.parametrize("n", [2049, 2100, 3000, 3073, 3100, 3500, 4096])
 def test_split_schedule_matches_the_oracle(n):
-    """Long query blocks split over two workgroups and merged by the last one to finish (a workspace is
-    given): rows on both sides of the split point and the last rows, against decode over i + 1 keys."""
+    """A workspace is given.  Beyond 3072 tokens long query blocks are split over two workgroups and merged by the
+    last one to finish; the shorter prompts run the wave form, which leaves the workspace alone.  Rows on both sides
+    of the split point and the last rows, against decode over i + 1 keys."""
     log(f"case: split prefill N={n}")
     ws = prefill_workspace(n)
     assert ws[1] > 0
@@ -122,17 +123,17 @@ def test_split_schedule_matches_the_oracle(n):
     sampled_rows_match_decode(out, qr, kr, vr, n, rows, f"split N={n}")
 
 
-def test_split_schedule_through_a_permuted_block_table():
-    """The split-K pair schedule (a workspace, N > 2048) over a permuted block table with spare blocks and a
-    ragged last block: cache rows through the table bit-exact, sampled rows on both sides of the split point
-    against decode over i + 1 keys."""
-    n, nb = 2500, 200
+@pytest.mark.parametrize("n,nb", [(2500, 200), (3300, 240)])
+def test_split_schedule_through_a_permuted_block_table(n, nb):
+    """A prompt with a workspace (2500 tokens: the wave form; 3300: the split-K pair schedule) over a permuted block
+    table with spare blocks and a ragged last block: cache rows through the table bit-exact, sampled rows on both
+    sides of the split point against decode over i + 1 keys."""
     log(f"case: split prefill through a permuted block table, N={n}, {nb} blocks")
     rng = np.random.default_rng(11)
     table = rng.permutation(nb)[:(n + 15) // 16].astype(np.int32)
     ws = prefill_workspace(n)
     assert ws[1] > 0
-    out, qr, kr, vr, scratch, q = run_prefill(n, seed=2500, table=table, num_blocks=nb, workspace=ws)
+    out, qr, kr, vr, scratch, q = run_prefill(n, seed=n, table=table, num_blocks=nb, workspace=ws)
     rows = [0, 15, 16, 1023, 1024, 2047, 2048, 2049, 2300, n - 17, n - 2, n - 1]
     sampled_rows_match_decode(out, qr, kr, vr, n, rows, f"split N={n} permuted table")
 
@@ -189,11 +190,12 @@ def test_config4_every_row_and_a_row_of_every_query_block(split):
     sampled_rows_match_decode(out, qr, kr, vr, n, rows, f"config4 split={split} oracle")
 
 
-@pytest.mark.parametrize("n,split", [(1100, False), (3000, True)])
+@pytest.mark.parametrize("n,split", [(1100, False), (3000, True), (3500, True), (4096, True)])
 def test_scores_rising_along_the_sequence_move_the_softmax_reference(n, split):
     """Keys whose scores grow by ~41 log2 units along the sequence: the running maximum of every query passes
     its exponent reference several times (the kernel rescales O and the row sums only when the maximum exceeds
-    the reference by 2^8), in both schedules, against decode over i + 1 keys."""
+    the reference by 2^8), in the wave form (up to 3072 tokens) and in the pair schedule with its merge of two parts,
+    against decode over i + 1 keys."""
     log(f"case: prefill rising scores N={n} split={split}")
     rng = np.random.default_rng(n)
     q = O.f32_to_f16((0.25 + 0.01 * rng.standard_normal(n * 2048)).astype(np.float32))

@@ -91,14 +91,15 @@ def test_a_step_of_minus_infinite_scores_has_weight_zero(n):
         check(run(n, f32, q, k, v), exact(q, k, v), f32, f"-inf step N={n} f32={f32}")
 
 
-def test_scores_rising_over_the_waves_steps():
-    """Scores that grow along the keys move every wave's softmax reference again and again."""
-    n = 1500
-    log(f"case: rising scores N={n}")
+@pytest.mark.parametrize("n,workspace", [(1500, False), (3500, True), (4096, True)])
+def test_scores_rising_over_the_waves_steps(n, workspace):
+    """Scores that grow along the keys move every wave's softmax reference again and again, and in the pair schedule
+    (3500 and 4096 tokens) leave the two parts of a block with references far apart."""
+    log(f"case: rising scores N={n} workspace={workspace}")
     q, k, v = operands(n, 99)
     import torch
     ramp = torch.linspace(0, 6, n, device="cuda").half()
     q[:, :, 1] = 12
     k[:, :, 1] = ramp[:, None] * 8
     for f32 in (False, True):
-        check(run(n, f32, q, k, v), exact(q, k, v), f32, f"rising N={n} f32={f32}")
+        check(run(n, f32, q, k, v, workspace), exact(q, k, v), f32, f"rising N={n} f32={f32}")

@@ -194,7 +194,7 @@ def test_prefill_then_decode_on_the_same_paged_cache(n, steps):
 
     def decode(pos, d_k, d_v, ragged=False):
         """One decode step at `pos`: a uniform length runs the single-shot kernel through the block table, a
-        ragged one (cache_lens given) the persistent kernel and the merge kernel."""
+        ragged one (cache_lens given, partitions of 512 tokens) the persistent kernel and the merge kernel."""
         out = torch.zeros(2048, dtype=torch.int16, device="cuda")
         wsb = pvlc.decode_workspace_bytes(1, total)
         ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
@@ -205,7 +205,8 @@ def test_prefill_then_decode_on_the_same_paged_cache(n, steps):
                                    value_cache=d_v, query=keep[0], new_key=keep[1], new_value=keep[2], out=out,
                                    workspace=ws, workspace_bytes=wsb, max_context=total, block_tables=d_table,
                                    cache_lens=keep[3] if ragged else None, uniform_cache_len=pos, rope_cos=d_cos,
-                                   rope_sin=d_sin, rope_rows=total, rotate_query=True)
+                                   rope_sin=d_sin, rope_rows=total, rotate_query=True,
+                                   partition_tokens=512 if ragged else 0)
         pvlc.paged_decode_f16(a)
         torch.cuda.synchronize()
         assert pvlc.workspace_error(ws, wsb) == 0

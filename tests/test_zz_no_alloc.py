@@ -2,9 +2,9 @@
 
 The no-alloc entry point runs the same kernels with the split-K state in the library's per-device scratch array;
 its outputs and caches must equal the workspace entry point's bit for bit, call after call, whatever the previous
-call left in the shared scratch: an 18-layer single-shot step (in-kernel merge through the counters), then smaller
-launches -- a ragged paged batch on the streaming kernel with an automatic partition (status words, merge kernel)
-and a 4-layer single-shot step whose counters are the ones the first call left.  Each call is also checked against
+call left in the shared scratch: an 18-layer single-shot step (in-kernel merge through the counters), then a ragged
+paged batch in one launch, another on the streaming kernel with an automatic partition (status words, merge kernel),
+and a 4-layer single-shot step whose counters are the ones the earlier calls left.  Each call is also checked against
 the oracle on a sampled sequence.  Launches beyond the scratch are rejected before any GPU effect.
 """
 
@@ -103,8 +103,11 @@ def check_pair(case, label):
 def test_no_alloc_matches_the_workspace_entry_point_call_after_call():
     log("case: no-alloc call 1: 18 layers, T=2048, single shot")
     check_pair(make_case(18, [2048] * 18, seed=31, paged=False), "no-alloc 18 layers T=2048")
-    log("case: no-alloc call 2 (smaller): 6 ragged paged sequences, automatic streaming partition")
+    log("case: no-alloc call 2 (smaller): 6 ragged paged sequences, one launch")
     check_pair(make_case(6, [700, 3100, 90, 1600, 2999, 17], seed=32, paged=True), "no-alloc ragged 6")
+    log("case: no-alloc: 40 ragged paged sequences, automatic streaming partition")
+    assert pvlc.decode_partition(40, 2000) == 512  # beyond the 384 tokens of one launch's workgroup
+    check_pair(make_case(40, [2000, 90, 1311, 17, 1024] * 8, seed=34, paged=True), "no-alloc ragged 40")
     log("case: no-alloc call 3 (smaller): 4 layers, T=300, single shot")
     check_pair(make_case(4, [300] * 4, seed=33, paged=False), "no-alloc 4 layers T=300")
 
