@@ -22,9 +22,12 @@ typedef u16x8_t u16x8_any __attribute__((aligned(2)));
 // a token) and the slabs (a wave on 1 KiB) move in 16-byte vectors on
 // contiguous runs on either side.  A thread per (token, head, chunk) without
 // LDS scattered the values 2 bytes at a time on the cache side.  They are
-// bound by latency for a few thousand tokens (loads, LDS, stores) and by HBM
+// bound by latency for a few thousand tokens (loads, LDS, stores) and by memory
 // beyond: 5003 tokens 13.1 -> 8.6 us for the pair of calls (two launches from
-// the host are 8.2 of it), 65536 tokens 84.8 -> 41.3 (6.5 TB/s).
+// the host are 8.2 of it), 65536 tokens, four prefixes in turn, 100.6 -> 47.2.
+// There a pack takes 27.2 us (4.9 TB/s, what a large copy reaches) and the pair
+// less than twice that, since the unpack finds part of the planes in the
+// Infinity Cache; one prefix over and over, which fits there, 84.9 -> 40.9.
 constexpr int kMoveThreads = 256;
 constexpr int kValuePad = 8;  // elements after each 256-dim LDS row, against bank conflicts
 

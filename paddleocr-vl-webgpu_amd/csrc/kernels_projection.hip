@@ -201,16 +201,17 @@ __device__ inline bool ordered_tile(const ProjectionOrder &o, uint32_t b, uint32
 // unit's load path moves lines: L2-resident reads of 16 rows x 64 bytes
 // measured 17 TB/s device-wide against 33 for 8 rows x 128 bytes (direct to
 // LDS or to registers alike), which bound the 128 x 256 and 128 x 160 tile
-// kernels this one replaced.  N=4096, split kernel included, before -> now:
-// q|k|v 55.8 -> 48.3 us, o 52.1 -> 44.8, gate|up 118 -> 93 (1.2 PFLOP/s of
-// MFMAs, the rate of a large bf16 library product on this card), down 69.0
-// -> 62.3.
+// kernels this one replaced.  N=4096, one projection repeated back to back
+// with its split kernel, before -> now: q|k|v 55-58 -> 48-50 us, o 50-51 -> 44-45,
+// gate|up 115-118 -> 93-94 (1.1 PFLOP/s of MFMAs, 1.2 without the split; a large
+// bf16 library product reaches 1.4), down 68-69 -> 62-63; the four in order,
+// whose activations come from further away, 318-322 -> 270-277.
 //
 // Small launches are bound by latency and by idle compute units, so their
 // tiles are small and the depth is split over KG groups, whose sums are added
 // through LDS in a fixed order (the result does not depend on timing).  211
-// rows: q|k|v 25.3 -> 13.2 us, o 35.8 -> 13.1, gate|up 26.0 -> 15.8, down
-// 47.0 -> 16.7; 16 rows: 18.6 -> 7.7, 29.0 -> 9.2, 18.4 -> 8.1, 40.1 -> 11.3.
+// rows: q|k|v 25.8 -> 13.5 us, o 36.2 -> 13.3, gate|up 26.9 -> 16.1, down
+// 47.3 -> 16.7; 16 rows: 18.5 -> 8.0, 29.0 -> 9.3, 18.4 -> 8.4, 40.4 -> 11.5.
 //
 // LDS slot layout [row][8 chunks of 8 k], chunk c of row r in place c ^ (r %
 // 8): a load's 8 lanes still read one line, and the 8 rows of a fragment read

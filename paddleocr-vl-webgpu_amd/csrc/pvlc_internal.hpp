@@ -291,8 +291,7 @@ int launch_linear_projection_f16(const float *input, const uint16_t *weight, con
 // storing its own part: config 4 at N=4096, 99.8-100.8 -> 96.6-97.3 us mean
 // per call.  The workspace is asked for when the longest block is longer than
 // kPrefillSplitSteps and used by prompts beyond kPrefillWaveTokens.  A pair
-// whose light workgroup
-// would take fewer than kPrefillSplitMin heavy steps at an even split is not
+// whose light workgroup would take fewer than kPrefillSplitMin heavy steps at an even split is not
 // split (the light block and the heavy block run whole on the two
 // workgroups): a second segment costs its workgroup a query load, a pipeline
 // fill and the partial hand-off, about what 4 to 5 steps cost (measured at

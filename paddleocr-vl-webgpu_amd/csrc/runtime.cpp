@@ -285,9 +285,10 @@ pvlc_hip_status launch_decode_state(const pvlc_hip_paged_decode_args *a, uint32_
     // workgroup per (partition, kv head, sequence), those past the end of
     // their sequence leaving at once: one launch instead of two, without the
     // persistent kernel's pass over all lengths.  2 to 256 sequences of up to
-    // 128 to 6000 rows, every spread of lengths (all equal, 1:4, 1:16): 6-14 us
-    // against 11.5-17 (13 sequences up to 2010 rows 8.6 against 13.6; 256 up
-    // to 300, 512 workgroups, 14.3-17.9 against 16.1-19.6).
+    // 128 to 6000 rows, every spread of lengths (all equal, 1:4, 1:16): 6-18 us
+    // against 11.5-20 (13 sequences up to 2010 rows 8.6 against 13.6; the
+    // longest launches, 256 up to 300 rows in 512 workgroups, 14.3-17.9
+    // against 16.1-19.6).
     const uint32_t part_tiles = (partition + kBlockTokens - 1) / kBlockTokens;
     const uint64_t workgroups = static_cast<uint64_t>(max_parts) * kKvHeads * a->num_seqs;
     const bool streaming = a->num_seqs <= kMaxRaggedSeqs &&
