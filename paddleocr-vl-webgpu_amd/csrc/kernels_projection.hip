@@ -17,8 +17,8 @@
 // 32-wide k step one 16 KiB block [plane][k-chunk (4)][row (128)][8]), so a
 // GEMM stage of the activations is one contiguous 16 KiB run.
 // Kernel 2 (GEMM): one template from 128 x 192 down to 16 x 16 output tiles;
-// the host picks the tile by a cost that counts, per compute unit, the matrix
-// time and the bytes through its load path (choose_projection_tile).  The waves of
+// the host picks the tile by the measured times of a compute unit's first tile
+// and its further ones (choose_projection_tile).  The waves of
 // a workgroup own rows of the tile (activation fragments straight from the
 // planes into registers, no byte read twice) and share its weight columns,
 // which move by direct global-to-LDS loads in whole 128-byte lines; small

@@ -197,14 +197,21 @@ inline ProjectionWorkspaceLayout projection_workspace_layout(uint32_t rows, uint
     const size_t tiles = padded * k_width * 4;  // two fp16 planes
     return {tiles, tiles + (padded * 4 + 255) / 256 * 256};
 }
-// The tiles of the projection GEMM (kernels_projection.hip) and the threads of
-// their workgroups, by preference on equal cost.
+// The tiles of the projection GEMM (kernels_projection.hip), the threads of
+// their workgroups, and the measured time of a compute unit's first tile and of
+// each further one (0.1 us at a depth of 1024; medians over 24 numbers of rows
+// from 8 to 4096 and ten pairs of widths, split kernel taken off), by preference
+// on equal cost.  Two workgroups of the larger tiles overlap on a unit, the
+// 512-thread group of 128 x 96 is alone there: its further tiles cost as much as
+// those of 128 x 128.  (128 x 128's first is 169 by the median; 172 leaves q|k|v of
+// 1025 to 1152 rows to two turns of 64 x 96, 1% faster for the layer.)
 struct ProjectionTile {
-    uint32_t rows, cols, threads;
+    uint32_t rows, cols, threads, first, next;
 };
-constexpr ProjectionTile kProjectionTiles[] = {{128, 192, 256}, {128, 160, 256}, {128, 128, 256}, {128, 64, 512},
-                                               {64, 64, 256},   {128, 96, 512},  {64, 96, 256},   {32, 64, 256},
-                                               {16, 64, 256},   {16, 32, 512},   {16, 16, 512}};
+constexpr ProjectionTile kProjectionTiles[] = {
+    {128, 192, 256, 228, 210}, {128, 160, 256, 200, 168}, {128, 128, 256, 172, 138}, {128, 64, 512, 105, 92},
+    {64, 64, 256, 82, 50},     {128, 96, 512, 134, 149},  {64, 96, 256, 101, 70},    {32, 64, 256, 66, 39},
+    {16, 64, 256, 54, 28},     {16, 32, 512, 50, 21},     {16, 16, 512, 49, 14}};
 constexpr int kProjectionTileCount = sizeof(kProjectionTiles) / sizeof(kProjectionTiles[0]);
 constexpr uint32_t kXcds = 8;           // MI355X: 8 XCDs, each with its own L2
 constexpr uint32_t kXcdUnits = 32;      // compute units of one XCD
@@ -239,16 +246,16 @@ inline ProjectionOrder projection_order(uint32_t row_tiles, uint32_t col_tiles, 
     return best;
 }
 
-// The tile of a launch: the least clocks of the busiest compute unit per
-// 32-deep step, (tiles it runs) x max(matrix time, load time) with rows cols /
-// 32 clocks of MFMAs (hi and lo, 4096 FLOP per clock) and 2 rows + cols clocks
-// of loads (64 bytes per clock) a tile; on ties the earlier in the list (two
-// 64 x 64 tiles a unit overlap, one 128 x 96 does not: 300 rows of gate|up 17.5
-// against 19.1 us).  The unit's tiles are those of the largest XCD block over
-// its 32 units.  Against every tile timed at 16 to 4096 rows of the decoder's
-// projections this picks the fastest or one within 3% of it.  What the 96
-// column tiles save over the others: 400 rows, gate|up 23.3 -> 20.9 us; 900
-// rows, q|k|v 23.5 -> 20.8; 1157 rows, o 26.1 -> 24.0 and down 33.0 -> 30.4.
+// The tile of a launch: the least time of the busiest compute unit, which runs
+// the tiles of the largest XCD block over the XCD's 32 units, by the measured
+// times of its first tile and the further ones.  Against every tile timed at
+// those rows and widths this picks the fastest or one within 6% of it, 0.2%
+// slower on average.  (Clocks of the matrix or load path by the tile's area in
+// place of measured times took 128 x 96 too often: 2500 rows of gate|up 87.3 us
+// against 67.9 with 128 x 128, 3500 rows 117.5 against 88.7 with 128 x 192, 1836
+// rows of 1152 to 4304 columns 55.4 against 46.7 with 128 x 160; where one turn
+// does, that tile saves: 400 rows, gate|up 23.3 -> 20.9 us; 900 rows, q|k|v 23.5
+// -> 20.8; 1157 rows, o 26.1 -> 24.0 and down 33.0 -> 30.4 with 64 x 96.)
 // The grid, 8 times the largest block, keeps under 2^32 threads, which few rows
 // of 2^30 or more columns exceed with the small tiles.  -1: no tile does.
 inline int choose_projection_tile(uint32_t rows, uint32_t k_width, uint32_t n_width, ProjectionOrder *order, uint64_t *block) {
@@ -262,8 +269,7 @@ inline int choose_projection_tile(uint32_t rows, uint32_t k_width, uint32_t n_wi
         if (i + 1 < kProjectionTileCount && (n_width < t.cols || k_width > 1u << 28)) continue;
         uint64_t b = 0;
         const ProjectionOrder o = projection_order(rows / t.rows + (rows % t.rows != 0), n_width / t.cols + (n_width % t.cols != 0), t, &b);
-        const uint64_t mfma = t.rows * t.cols / 32, loads = 2 * t.rows + t.cols;
-        const uint64_t cost = (b + kXcdUnits - 1) / kXcdUnits * (mfma > loads ? mfma : loads);
+        const uint64_t turns = (b + kXcdUnits - 1) / kXcdUnits, cost = t.first + (turns - 1) * t.next;
         if (cost < best_cost && b * kXcds * t.threads < 1ull << 32) {
             best_cost = cost;
             best = i;

@@ -1,6 +1,7 @@
 """The tile that the projection chooses (csrc/pvlc_internal.hpp): for every admitted geometry whose operands a device of up
 to 512 GiB could hold, a tile is found, its grid stays under 2^32 threads, its weight offsets within 32 bits, and its
-blocks cover every output tile; few rows of very many columns among them."""
+blocks cover every output tile; few rows of very many columns among them.  And the tiles that were measured fastest where
+the choice is between sizes far apart."""
 
 import os
 import shutil
@@ -44,6 +45,18 @@ int main() {
     for (uint64_t n = 1ull << 29; n < 1ull << 31; n += (1ull << 25) + 4)
         for (uint64_t rows : {1, 8, 16, 17, 32, 64, 128}) check(rows, 32, n);
     for (uint64_t rows : {1, 16, 4096, 8388479, 8388480}) for (uint64_t n : {4, 12, 16, 28, 32, 60, 64, 124, 128, 188, 192}) check(rows, 32, n);
+    // rows, k, n; the fastest tile of all, and its lead over 128 x 96
+    const uint32_t fastest[][5] = {{2500, 1024, 6144, 128, 128},   // 67.9 us against 87.3
+                                   {3500, 1024, 6144, 128, 192},   // 88.7 against 117.5
+                                   {1300, 1024, 6144, 128, 160},   // 41.7 against 51.3
+                                   {1836, 1152, 4304, 128, 160},   // 46.7 against 55.4
+                                   {2500, 1152, 3456, 128, 160}};  // 48.9 against 59.9
+    for (const auto &f : fastest) {
+        ProjectionOrder o{};
+        uint64_t block = 0;
+        const ProjectionTile t = kProjectionTiles[choose_projection_tile(f[0], f[1], f[2], &o, &block)];
+        if (t.rows != f[3] || t.cols != f[4]) std::printf("%u x %u x %u takes %u x %u\n", f[0], f[1], f[2], t.rows, t.cols), ++fails;
+    }
     for (int i = 0; i < kProjectionTileCount; ++i) if (!seen[i]) { std::printf("tile %d never chosen\n", i); ++fails; }
     std::printf("%d geometries, %d failures\n", checks, fails);
     return fails != 0;
